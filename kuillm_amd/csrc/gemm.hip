@@ -9,11 +9,16 @@
 // __shared__ array so the compiler need not make LDS reads wait for DMA that
 // targets the other stage.
 //
-// Everything else bf16 / f16 (any M, N; K % 8 == 0): `gemm_mfma_kernel` --
-// BM x BN x 64 tiles (256x256 or 128x128), 4 waves, register-staged global
-// loads (a row-major B is transposed in registers on its way into LDS), two
-// LDS stages, optional split-K whose fp32 partials `splitk_reduce_kernel`
-// sums in split order (deterministic).
+// Smaller and ragged bf16 / f16 GEMMs (any M, N; K % 8 == 0):
+// `gemm_tile_kernel` (gemm_tile.hpp) -- output tiles from 64x64 to 128x256
+// chosen by a cost model (choose_tile), three or four LDS-DMA stages,
+// optional split-K whose fp32 partials `splitk_reduce_kernel` sums in split
+// order (deterministic).
+//
+// Operands past 31-bit buffer offsets: `gemm_mfma_kernel` -- 128x128x64
+// tiles, 4 waves, register-staged global loads with 64-bit addresses (a
+// row-major B is transposed in registers on its way into LDS), two LDS
+// stages.
 //
 // Work-group ids are remapped so that neighbouring output tiles run on the
 // same XCD (dispatch is round-robin over the 8 XCDs, each with its own L2)
@@ -28,24 +33,9 @@
 
 #include <type_traits>
 
-#include "common.hpp"
+#include "gemm_tile.hpp"
 
 namespace kuiops {
-
-struct GemmArgs {
-    int64_t M, N, K;
-    const void *A; int64_t lda, stride_a;
-    const void *B; int64_t ldb, stride_b;
-    void *out; int64_t ldo, stride_o;
-    const void *cin; int64_t ldcin; int c_kind;
-    float alpha, beta;
-    int64_t k_per_split;   // multiple of 64
-    int splits;
-    int tiles_m, tiles_n;
-    int vec_store;         // gemm_dma_kernel: 16-byte row-segment epilogue (ldo, N % 8 == 0, aligned out)
-    int raster;            // tile order within a batch entry: 0 = groups of 8 tile-rows, 1 = row by row
-    float *partial;        // split-K workspace [splits][M][N]
-};
 
 __device__ __forceinline__ int swz(int row) { return (row ^ (row >> 3)) & 7; }
 
@@ -62,34 +52,6 @@ __device__ __forceinline__ void tile_coords(int bid, int nblocks, int tiles_m, i
     const int first_m = group * G;
     const int gsz = min(tiles_m - first_m, G);
     const int in_group = pid - group * width;
-    tm = first_m + in_group % gsz;
-    tn = in_group / gsz;
-}
-
-// Batched form: the linear id runs over batch x tiles; after the XCD remap
-// each batch entry's tiles are contiguous (so one XCD's L2 holds its A and
-// B), and tiles are grouped by 8 tile-rows within the entry.
-__device__ __forceinline__ void tile_coords_batched(int bid, int nblocks, int tiles_m, int tiles_n,
-                                                    int &tm, int &tn, int &bz, int raster = 0) {
-    const int xcd = bid & 7, idx = bid >> 3;
-    const int q = nblocks >> 3, r = nblocks & 7;
-    const int pid = xcd * q + (xcd < r ? xcd : r) + idx;
-    const int per = tiles_m * tiles_n;
-    bz = pid / per;
-    const int t = pid - bz * per;
-    if (raster) {
-        // row by row: the tiles one XCD runs at once lie side by side, so
-        // their 512-byte row segments of the output form whole rows
-        tm = t / tiles_n;
-        tn = t - tm * tiles_n;
-        return;
-    }
-    const int G = 8;
-    const int width = G * tiles_n;
-    const int group = t / width;
-    const int first_m = group * G;
-    const int gsz = min(tiles_m - first_m, G);
-    const int in_group = t - group * width;
     tm = first_m + in_group % gsz;
     tn = in_group / gsz;
 }
@@ -289,36 +251,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
 // rows / columns past M / N are clamped on load and dropped on store.
 __device__ __forceinline__ int swzB(int k) { return ((k & 3) | (((k >> 3) & 1) << 2)) << 2; }
 
-typedef __attribute__((address_space(3))) char lds_char;
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-// Generic -> LDS address-space cast.  A direct cast keeps the pointer's
-// provenance (an integer round trip would hide which LDS array it points
-// into, and the compiler would then make every LDS read wait for all
-// in-flight LDS-DMA loads).
-__device__ __forceinline__ lds_char *to_lds(const void *p) {
-    return (lds_char *)(const_cast<void *>(p));
-}
-
-// One global_load_lds_dwordx4: 16 bytes from `src` per lane into
-// dst + 16 * lane (dst is wave-uniform).  The source must reach the builtin
-// as `const void *`: a typed pointer makes the host compilation pass drop
-// the kernel's launch stub without a diagnostic.
-__device__ __forceinline__ void dma16(const void *src, const void *dst) {
-    __builtin_amdgcn_global_load_lds(src, to_lds(dst), 16, 0, 0);
-}
-
-// Buffer-resource form of the same copy: a wave-uniform descriptor (SGPRs),
-// a per-lane 32-bit byte offset and a uniform byte offset, so the K-step
-// advance costs no per-lane address registers.  Reads past `bytes` return 0.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, const void *dst) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)to_lds(dst), 16,
-                                             (int)voff, (int)soff, 0, 0);
-}
-
 // Epilogue of one 32x32 accumulator tile: lane holds column `col` and rows
 // row0 + 8 * (e / 4) + 4 * lk + e % 4.  The addend kind is wave-uniform.
 template <typename Tout>
@@ -349,13 +281,6 @@ __device__ __forceinline__ void store_tile32(const GemmArgs &a, const f32x16 &ac
         const int r = (e >> 2) * 8 + lk * 4 + (e & 3);
         if (full_rows || row0 + r < a.M) out[(int64_t)r * a.ldo] = from_f32<Tout>(a.alpha * acc[e] + add[e]);
     }
-}
-
-// vmcnt-only wait (expcnt / lgkmcnt left at their maxima), N < 64.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt out of range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
 template <typename T, bool BCOL, typename Tout, int WM, int WN, int BK, int NS>
@@ -584,14 +509,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_dma_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
             store_tile32<Tout>(a, acc[i][j], m0 + wm * WTM + i * 32, n0 + wn * WTN + j * 32 + lrow, lk);
-}
-
-// Uniform (wave-invariant) pointer kept in SGPRs: buffer descriptors built
-// from it need no per-lane waterfall loop around each DMA.
-__device__ __forceinline__ const char *uniform_ptr(const char *p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
 }
 
 // ------------------------------------------------------------------------
@@ -1137,20 +1054,6 @@ void gemm_wave_kernel(GemmArgs a) {
     }
 }
 
-// Sums split-K partials in split order, then applies alpha / beta / addend.
-template <typename Tout>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs a) {
-    const int64_t total = a.M * a.N;
-    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total;
-         idx += (int64_t)gridDim.x * 256) {
-        float s = 0.f;
-        for (int z = 0; z < a.splits; ++z) s += a.partial[(int64_t)z * total + idx];
-        const int64_t row = idx / a.N, col = idx - row * a.N;
-        epilogue_store<Tout>(a, reinterpret_cast<Tout *>(a.out), reinterpret_cast<const Tout *>(a.cin),
-                             row, col, s);
-    }
-}
-
 // Generic LDS-tiled SIMT GEMM (any strides / shapes / float dtypes): 64x64
 // tile, 256 threads each owning a 4x4 strided patch, K step 16.
 template <typename Tin, typename Tacc, typename Tout>
@@ -1215,39 +1118,89 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(GemmArgs a, int b_col) {
 
 // ------------------------------------------------------------ host dispatch
 
-struct TileCfg { int bm, bn; };
-
-static TileCfg pick_tile(int64_t M, int64_t N, int64_t batch) {
-    // 256x256 tiles only when they still give a full wave of work-groups.
-    if (M >= 2048 && N >= 2048 && cdiv(M, 256) * cdiv(N, 256) * batch >= 192) return {256, 256};
-    return {128, 128};
-}
-
-static int choose_splits(int64_t M, int64_t N, int64_t K, int64_t batch, TileCfg t) {
-    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
-    if (batch != 1 || tiles >= 128 || K < 1024) return 1;
+// Largest split count of an M x N x K product (batch 1): the workspace query's
+// bound.  Splits are for grids that leave CUs idle over a long K.
+static int max_splits(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = cdiv(M, 128) * cdiv(N, 128);
+    if ((M >= 2048 && N >= 2048 && cdiv(M, 256) * cdiv(N, 256) >= 192) || tiles >= 128 || K < 1024) return 1;
     int64_t s = cdiv(256, tiles);
     s = s < (K / 512) ? s : (K / 512);
     if (s > 16) s = 16;
     return s < 1 ? 1 : (int)s;
 }
 
+// gemm_tile_kernel's output tiles.  A CU keeps about 32 KB of loads in flight
+// whatever the kernel asks for, which at the latency of HBM and the MALL is
+// 50 to 60 GB/s, so a tile's time is its bytes ((BM + BN) * 128 per 64 k) over
+// that rate, not its MFMAs, until 128 x 256.  Measured per stage with the
+// weights streaming from HBM (us): 64 x 64 0.29 (one work-group per CU) and
+// 0.23 (several), 128 x 64 0.79 for 128 k, 128 x 128 0.59, 128 x 192 0.80,
+// 128 x 256 0.93.  Measured at 512 x N x K (bf16, nn.Linear weights cold in
+// HBM; the register-staged 128 x 128 tiles that ran here before, and this
+// choice): 11264 x 2048 47 -> 31.5 us, 2048 x 2048 30 -> 11.9, 2048 x 5632
+// 33 -> 27; 203 x 4864 x 896 24.9 -> 9.7.
+struct TileCfg { int bm, bn, bk; float stage, stage_many; };
+static const TileCfg kTiles[] = {
+    {64, 64, 64, 0.285f, 0.23f}, {128, 64, 128, 0.79f, 0.86f}, {128, 128, 64, 0.59f, 0.59f},
+    {128, 192, 64, 0.80f, 0.78f}, {128, 256, 64, 0.93f, 0.95f}};
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+struct TileChoice { int tile, splits; float us; };
+
+// The tile and split count of least estimated time: rounds of one tile per
+// CU, and for a split the partials' traffic plus the second launch.  max_s
+// bounds the splits; fixed_s > 0 asks for that many.
+static TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int max_s, int fixed_s) {
+    TileChoice best{0, 1, 1e30f};
+    const int64_t cus = num_cus();
+    for (int t = 0; t < kNumTiles; ++t) {
+        const TileCfg &c = kTiles[t];
+        const int64_t tiles = cdiv(M, c.bm) * cdiv(N, c.bn) * batch;
+        for (int s = fixed_s > 0 ? fixed_s : 1; s <= (fixed_s > 0 ? fixed_s : max_s); ++s) {
+            const int64_t rounds = cdiv(tiles * s, cus);
+            const int64_t stages = cdiv(cdiv(K, s), c.bk);
+            float us = 2.2f + (float)rounds * ((float)stages * (rounds > 1 ? c.stage_many : c.stage) + (rounds > 1 ? 2.f : 0.f));
+            if (s > 1) us += 4.f + (float)s * (float)(M * N) * 8.f / 6e6f;
+            if (us < best.us) best = {t, s, us};
+        }
+    }
+    return best;
+}
+
 template <typename T, typename Tout, bool SPLIT>
-static void launch_mfma(const GemmArgs &a, TileCfg t, bool bcol, int64_t gz, hipStream_t st) {
-    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
-    dim3 grid((unsigned)tiles, (unsigned)gz);
-#define KUIOPS_GEMM_LAUNCH(BM, BN, WM, WN)                                                        \
-    do {                                                                                          \
-        if (bcol)                                                                                 \
-            hipLaunchKernelGGL((gemm_mfma_kernel<T, BM, BN, WM, WN, true, Tout, SPLIT>), grid,    \
-                               dim3(WM * WN * 64), 0, st, a);                                     \
-        else                                                                                      \
-            hipLaunchKernelGGL((gemm_mfma_kernel<T, BM, BN, WM, WN, false, Tout, SPLIT>), grid,   \
-                               dim3(WM * WN * 64), 0, st, a);                                     \
+static void launch_tile(int tile, const GemmArgs &a, bool bcol, dim3 grid, hipStream_t st) {
+#define KUIOPS_TILE_LAUNCH(WM, WN, WK, TM, TN, NS)                                                             \
+    do {                                                                                                       \
+        if (bcol)                                                                                              \
+            hipLaunchKernelGGL((gemm_tile_kernel<T, true, Tout, WM, WN, WK, TM, TN, NS, SPLIT>), grid,         \
+                               dim3(WM * WN * WK * 64), 0, st, a);                                             \
+        else                                                                                                   \
+            hipLaunchKernelGGL((gemm_tile_kernel<T, false, Tout, WM, WN, WK, TM, TN, NS, SPLIT>), grid,        \
+                               dim3(WM * WN * WK * 64), 0, st, a);                                             \
     } while (0)
-    if (t.bm == 256) KUIOPS_GEMM_LAUNCH(256, 256, 2, 2);
-    else KUIOPS_GEMM_LAUNCH(128, 128, 2, 2);
-#undef KUIOPS_GEMM_LAUNCH
+    switch (tile) {
+        case 0: KUIOPS_TILE_LAUNCH(2, 2, 1, 1, 1, 4); break;
+        case 1: KUIOPS_TILE_LAUNCH(2, 2, 2, 2, 1, 3); break;
+        case 2: KUIOPS_TILE_LAUNCH(2, 4, 1, 2, 1, 4); break;
+        case 3: KUIOPS_TILE_LAUNCH(2, 2, 1, 2, 3, 3); break;
+        default: KUIOPS_TILE_LAUNCH(2, 4, 1, 2, 2, 3); break;
+    }
+#undef KUIOPS_TILE_LAUNCH
+}
+
+template <typename Tout>
+static void launch_reduce(const GemmArgs &a, hipStream_t st) {
+    const bool vec = a.N % 4 == 0 && a.ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(a.out) & (4 * sizeof(Tout) - 1)) == 0;
+    const int64_t by = cdiv(a.M, 4);
+    const dim3 grid((unsigned)cdiv(a.N, vec ? 256 : 64), (unsigned)(by < 65535 ? by : 65535));
+    if (vec) hipLaunchKernelGGL((splitk_reduce_kernel<Tout, true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((splitk_reduce_kernel<Tout, false>), grid, dim3(256), 0, st, a);
+}
+
+template <typename T, typename Tout, bool SPLIT>
+static void launch_mfma(const GemmArgs &a, bool bcol, int64_t gz, hipStream_t st) {
+    dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n), (unsigned)gz);
+    if (bcol) hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 2, 2, true, Tout, SPLIT>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 2, 2, false, Tout, SPLIT>), grid, dim3(256), 0, st, a);
 }
 
 // KUIOPS_GEMM_KERNEL=dma selects the 8-wave gemm_dma_kernel for the large
@@ -1261,11 +1214,14 @@ static int gemm_kernel_choice() {
     return choice;
 }
 
-static bool dma_eligible(const GemmArgs &a, int64_t batch, bool bcol) {
-    // buffer offsets (tile rows x leading dim + K) must stay below 2^31 bytes
+// Buffer offsets (tile rows x leading dim + K) must stay below 2^31 bytes.
+static bool offsets_fit(const GemmArgs &a, bool bcol) {
     const int64_t lim = (int64_t)1 << 30;
-    if ((256 * a.lda + a.K) >= lim) return false;
-    if (bcol ? (256 * a.ldb + a.K) >= lim : (a.K * a.ldb + 256) >= lim) return false;
+    return 256 * a.lda + a.K < lim && (bcol ? 256 * a.ldb + a.K : a.K * a.ldb + 256) < lim;
+}
+
+static bool dma_eligible(const GemmArgs &a, int64_t batch, bool bcol) {
+    if (!offsets_fit(a, bcol)) return false;
     // batched operands: the addend (addmm only) is not batched
     if (batch > 1 && (a.c_kind != KUIOPS_C_NONE || a.stride_a % 8 || a.stride_b % 8)) return false;
     return a.K % 128 == 0 && a.K > 0 && a.M >= 256 && a.N >= 256 &&
@@ -1297,7 +1253,21 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *
             return launch_status();
         }
     }
-    if (splits_req <= 1 && dma_eligible(a, batch, bcol)) {
+    // splits_req = 0 leaves the split count to choose_tile, as far as the
+    // workspace goes that max_splits asks for.
+    const bool ws_ok = ws && aligned16(ws);
+    const int max_s = batch == 1 ? max_splits(a.M, a.N, a.K) : 1;
+    const size_t part = (size_t)a.M * a.N * sizeof(float);
+    if (splits_req == 0 && max_s > 1 && (!ws || ws_bytes < (size_t)max_s * part)) return KUIOPS_E_WORKSPACE;
+    const TileChoice tc = choose_tile(a.M, a.N, a.K, batch, ws_ok ? max_s : 1,
+                                      batch == 1 ? splits_req : 1);
+    // The 256x256 tiles run 1.45 us per 64 k and about 5 us around them, one
+    // per CU: with 128 of them (2048 x 4096 outputs) half the CUs idle and
+    // 128 x 256 tiles finish first (K = 4096: 60 against 98 us), with 256 or
+    // more they win (4096^3: 98 against 122 us).
+    const int64_t tiles256 = cdiv(a.M, 256) * cdiv(a.N, 256) * batch;
+    const float us256 = 2.2f + (float)cdiv(tiles256, num_cus()) * ((float)(a.K / 64) * 1.45f + 3.f);
+    if (splits_req <= 1 && dma_eligible(a, batch, bcol) && (gemm_kernel_choice() == 1 || a.K < 512 || us256 <= tc.us)) {
         a.tiles_m = (int)cdiv(a.M, 256);
         a.tiles_n = (int)cdiv(a.N, 256);
         const int vec = sizeof(Tout) == 2 ? 8 : 4;    // elements per vector store
@@ -1326,29 +1296,36 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *
         }
         return launch_status();
     }
-    TileCfg t = pick_tile(a.M, a.N, batch);
-    a.tiles_m = (int)cdiv(a.M, t.bm);
-    a.tiles_n = (int)cdiv(a.N, t.bn);
-    int splits = splits_req > 0 ? splits_req : choose_splits(a.M, a.N, a.K, batch, t);
+    const bool tile_ok = a.K > 0 && offsets_fit(a, bcol);
+    const int bk = tile_ok ? kTiles[tc.tile].bk : 64, bm = tile_ok ? kTiles[tc.tile].bm : 128,
+              bn = tile_ok ? kTiles[tc.tile].bn : 128;
+    int splits = tile_ok ? tc.splits : (splits_req > 0 ? splits_req : max_s);
     if (batch != 1) splits = 1;
-    int64_t kps = cdiv(cdiv(a.K, splits), 64) * 64;
-    splits = (int)cdiv(a.K, kps);
-    if (splits <= 1) {
-        a.splits = 1;
-        a.k_per_split = cdiv(a.K, 64) * 64;
-        if (a.K == 0) a.k_per_split = 64;
-        launch_mfma<T, Tout, false>(a, t, bcol, batch, st);
-        return launch_status();
-    }
-    const size_t need = (size_t)splits * a.M * a.N * sizeof(float);
-    if (!ws || ws_bytes < need) return KUIOPS_E_WORKSPACE;
+    a.tiles_m = (int)cdiv(a.M, bm);
+    a.tiles_n = (int)cdiv(a.N, bn);
+    const int64_t kps = cdiv(cdiv(a.K, splits), bk) * bk;
+    splits = kps > 0 ? (int)cdiv(a.K, kps) : 1;
     a.splits = splits;
-    a.k_per_split = kps;
-    a.partial = reinterpret_cast<float *>(ws);
-    launch_mfma<T, Tout, true>(a, t, bcol, splits, st);
-    int64_t blocks = cdiv(a.M * a.N, 256);
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(splitk_reduce_kernel<Tout>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+    a.k_per_split = kps > 0 ? kps : 64;
+    if (splits > 1) {
+        if (!ws || ws_bytes < splits * part) return KUIOPS_E_WORKSPACE;
+        a.partial = reinterpret_cast<float *>(ws);
+    }
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
+    if (tile_ok && tiles * batch < INT32_MAX) {
+        // vector stores: 16 bytes of the output, or of the fp32 partials
+        if (splits > 1) a.vec_store = a.N % 4 == 0 && aligned16(ws);
+        else if (sizeof(Tout) == 4) a.vec_store = a.ldo % 4 == 0 && a.stride_o % 4 == 0 && aligned16(a.out);
+        else a.vec_store = a.N % 8 == 0 && a.ldo % 8 == 0 && a.stride_o % 8 == 0 && aligned16(a.out);
+        const dim3 grid((unsigned)(tiles * batch), (unsigned)splits);
+        if (splits > 1) launch_tile<T, Tout, true>(tc.tile, a, bcol, grid, st);
+        else launch_tile<T, Tout, false>(tc.tile, a, bcol, grid, st);
+    } else if (splits > 1) {
+        launch_mfma<T, Tout, true>(a, bcol, splits, st);
+    } else {
+        launch_mfma<T, Tout, false>(a, bcol, batch, st);
+    }
+    if (splits > 1) launch_reduce<Tout>(a, st);
     return launch_status();
 }
 
@@ -1397,10 +1374,8 @@ static int gemm_entry(GemmArgs a, int64_t batch, int in_dt, int out_dt, int b_la
 }
 
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    TileCfg t = pick_tile(M, N, 1);
-    int s = choose_splits(M, N, K, 1, t);
-    if (s <= 1) return 0;
-    return (size_t)s * M * N * sizeof(float);
+    const int s = max_splits(M, N, K);
+    return s <= 1 ? 0 : (size_t)s * M * N * sizeof(float);
 }
 
 }  // namespace kuiops

@@ -137,6 +137,42 @@ def test_addmm_wave_kernel_edges(cuda, layout, M, N, K, kind):
     assert_tol(out, O.addmm(npy(C), npy(A), npy(B), alpha, beta), torch.bfloat16)
 
 
+# One shape per output tile of the tile kernel (64x64, 128x64, 128x128,
+# 128x192, 128x256), each with ragged last tiles, K remainders of 8 .. 56 and
+# fewer, as many or more K steps than LDS stages; split K (130 x 384, 5 K
+# ranges); an output whose rows are not 16-byte aligned (N = 1003).
+TILE_SHAPES = [(65, 136, 8), (200, 520, 264), (300, 5000, 1032), (1000, 4000, 200), (500, 11264, 136),
+               (2100, 4104, 216), (130, 384, 2568), (257, 1003, 1160)]
+
+
+@pytest.mark.parametrize("layout", ["row", "col"])
+@pytest.mark.parametrize("M,N,K", TILE_SHAPES)
+def test_addmm_tile_kernel_edges(cuda, layout, M, N, K):
+    """Bias and full addends, fp32 output, both B layouts.  |error| <= half a
+    bf16 ulp (2^-9 |ref|) plus fp32 sums of K products of size ~0.05
+    (K * 2^-24 * 0.2 < 1e-4), inside the file's 1e-2."""
+    if layout == "row" and N % 8:
+        pytest.skip("row-major B of odd width is another kernel")
+    A, B = gen((M, K), torch.bfloat16, seed=51), gen((K, N), torch.bfloat16, 0.05, seed=52)
+    bias, C = gen((N,), torch.bfloat16, seed=53), gen((M, N), torch.bfloat16, seed=54)
+    Bd = B.to(cuda) if layout == "row" else B.t().contiguous().to(cuda).t()
+    ref = O.mm(npy(A), npy(B))
+    assert_tol(ops.addmm(bias.to(cuda), A.to(cuda), Bd), ref + npy(bias), torch.bfloat16)
+    assert_tol(ops.addmm(C.to(cuda), A.to(cuda), Bd, beta=2.0, alpha=0.5), 0.5 * ref + 2 * npy(C), torch.bfloat16)
+    o32 = ops.mm(A.to(cuda), Bd, out_dtype=torch.float32)
+    np.testing.assert_allclose(npy(o32), ref, rtol=2e-3, atol=2e-3)
+
+
+def test_mm_rows_past_buffer_offsets(cuda):
+    """A row-major B whose rows lie 32 MiB apart (offsets past 2^31 bytes)."""
+    M, N, K, ld = 130, 64, 72, 1 << 24
+    A, B = gen((M, K), torch.bfloat16, seed=55), gen((K, N), torch.bfloat16, 0.05, seed=56)
+    store = torch.empty((K - 1) * ld + N, dtype=torch.bfloat16, device=cuda)
+    Bd = store.as_strided((K, N), (ld, 1))
+    Bd.copy_(B.to(cuda))
+    assert_tol(ops.mm(A.to(cuda), Bd), O.mm(npy(A), npy(B)), torch.bfloat16)
+
+
 @pytest.mark.parametrize("layout", ["row", "col"])
 def test_mm_wave_kernel_f32_out(cuda, layout):
     """bf16 operands, fp32 output, on the large-tile kernel (ragged N)."""
