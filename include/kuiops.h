@@ -99,7 +99,7 @@ KUIOPS_API const char *kuiops_status_string(int status);
  *   TOPK:         a = rows, b = row length, c = k
  *   DECODE_ROWS_BATCHED: a = M, b = N, c = K
  * Workspace contents need no initialisation, except GEMV_SPLITK's first
- * 16 KB (arrival counters): zero before the first call, and every call
+ * 16 KB and SDPA_DECODE's first 64 KB (arrival counters): zero before the first call, and every call
  * leaves them zero.  Calls that share one workspace must be ordered on one
  * stream.                                                                  */
 KUIOPS_API size_t kuiops_query_workspace(int op, int64_t a, int64_t b, int64_t c);
@@ -249,7 +249,7 @@ KUIOPS_API int kuiops_sdpa_general(int64_t n, int64_t hq, int64_t hkv, int64_t l
  * kernel runs: a decode step recorded once in a HIP graph passes s = cache
  * capacity and advances kv_len on the device.  Requires the workspace of
  * kuiops_query_workspace(KUIOPS_OP_SDPA_DECODE, n*hq*l, s, ev), 16-byte
- * aligned, whose first bytes hold the split arrival counters: they must be
+ * aligned, whose first 64 KB hold the split arrival counters: they must be
  * zero before the first call and every call leaves them zero (calls that
  * share a workspace must not overlap).  One launch: the last split
  * work-group of each query-row group merges the splits.  Rows with no

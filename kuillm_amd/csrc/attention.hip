@@ -661,13 +661,18 @@ static int64_t decode_chunk_for(int64_t s, int64_t groups) {
     return c < decode_chunk(s) ? decode_chunk(s) : c;
 }
 
-// Workspace: split arrival counters (one per work-group row group, at most
-// one per query row; zero between calls), then the split states.
-static size_t decode_counter_bytes(int64_t rows) { return (size_t)cdiv(rows * 4 * kAttnCounterStride, 256) * 256; }
+// Workspace: split arrival counters (one per row group, zero between calls),
+// then the split states.  The counters have a fixed head region that no call
+// uses for anything else: calls of different shapes share one workspace, and
+// a region sized by the call's rows would put one call's states where another
+// one's counters are.  Row groups are only split while there are fewer than
+// two per CU, so the region holds a counter for each.
+constexpr int64_t kMaxSplitGroups = 1024;
+constexpr size_t kDecodeCounterBytes = kMaxSplitGroups * 4 * kAttnCounterStride;     // 64 KB
 
 size_t decode_workspace_bytes(int64_t rows, int64_t kv_len, int64_t ev) {
     const int64_t splits = cdiv(kv_len > 0 ? kv_len : 1, decode_chunk(kv_len));
-    return decode_counter_bytes(rows) + (size_t)rows * splits * (ev + 2) * sizeof(float) + 256;
+    return kDecodeCounterBytes + (size_t)rows * splits * (ev + 2) * sizeof(float) + 256;
 }
 
 template <typename T, int HD>
@@ -744,7 +749,7 @@ static int launch_decode(AttnArgs a, hipStream_t st) {
     // The last split work-group of a row group merges the splits in-kernel
     // (one launch) when there are few; with many, each split work-group
     // would wait for its write-through stores, so a second kernel merges.
-    const bool fused = a.splits <= kFusedMergeMaxSplits;
+    const bool fused = a.splits <= kFusedMergeMaxSplits && a.n * a.hkv * a.row_groups <= kMaxSplitGroups;
     if (!fused) a.counters = nullptr;
     switch (R) {
         // one or two rows: 8 keys per lane group, so a split of up to 128
@@ -833,11 +838,11 @@ extern "C" int kuiops_sdpa_decode(int64_t n, int64_t hq, int64_t hkv, int64_t l,
     a.splits = (int)cdiv(ss, a.chunk);
     const int64_t rows = n * hq * l;
     const size_t need = decode_workspace_bytes(rows, s, ev);
-    if ((int64_t)(need - decode_counter_bytes(rows)) >= INT32_MAX) return KUIOPS_E_UNSUPPORTED;  // 32-bit offsets
+    if ((int64_t)(need - kDecodeCounterBytes) >= INT32_MAX) return KUIOPS_E_UNSUPPORTED;  // 32-bit offsets
     if (!workspace || workspace_bytes < need) return KUIOPS_E_WORKSPACE;
     if (!aligned16(workspace)) return KUIOPS_E_WORKSPACE;
     a.counters = reinterpret_cast<unsigned *>(workspace);
-    a.ws_ml = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + decode_counter_bytes(rows));
+    a.ws_ml = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + kDecodeCounterBytes);
     a.ws_o = a.ws_ml + rows * a.splits * 2;
     if ((reinterpret_cast<uintptr_t>(a.ws_o) & 15) != 0) {
         // keep o rows 16-byte aligned

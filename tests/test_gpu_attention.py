@@ -204,6 +204,18 @@ def test_sdpa_decode_vs_oracle(cuda, n, hq, hkv, l, s, d):
     assert torch.equal(out, again)
 
 
+def test_sdpa_decode_shapes_share_workspace(cuda):
+    """Split calls of few and of many query rows in turn on one stream: no
+    call's split states may land on another one's arrival counters."""
+    calls = []
+    for i, (n, s) in enumerate([(1, 4096), (8, 2000), (1, 900), (16, 1500)]):
+        q, k, v = gen((n, 32, 1, 64), seed=31 + i), gen((n, 8, s, 64), seed=41 + i), gen((n, 8, s, 64), seed=51 + i)
+        calls.append(([t.to(cuda) for t in (q, k, v)], O.sdpa(npy(q), npy(k), npy(v))[0]))
+    for _ in range(2):
+        for args, ref in calls:
+            close(ops.sdpa(*args)[0], ref)
+
+
 def test_sdpa_decode_empty_keys(cuda):
     """No visible keys.  A batch entry whose device kv_len is 0, on the
     split kernel over a 4096-key cache (its K / V loads are issued before the
