@@ -15,17 +15,17 @@
 // optional split-K whose fp32 partials `splitk_reduce_kernel` sums in split
 // order (deterministic).
 //
-// Operands past 31-bit buffer offsets: `gemm_mfma_kernel` -- 128x128x64
-// tiles, 4 waves, register-staged global loads with 64-bit addresses (a
-// row-major B is transposed in registers on its way into LDS), two LDS
-// stages.
+// Operands of odd strides, sizes and alignments, or past 31-bit buffer
+// offsets: `gemm_mfma_kernel` -- 128x128x64 tiles, 4 waves, register-staged
+// global loads with 64-bit addresses (a row-major B is transposed in registers
+// on its way into LDS), two LDS stages.
 //
 // Work-group ids are remapped so that neighbouring output tiles run on the
 // same XCD (dispatch is round-robin over the 8 XCDs, each with its own L2)
 // and are visited in groups of 8 tile-rows.
 //
-// f32 / f64 and unaligned operands take `gemm_simt_kernel`, a plain
-// LDS-tiled kernel with the same epilogue.
+// f32 / f64 operands take `gemm_simt_kernel`, a plain LDS-tiled kernel with
+// the same epilogue.
 //
 // Semantics follow aten mm / addmm / bmm (the reference's fallthrough and
 // test oracle, kuipy/kuiops.py:403-564, tests/test_jit_ops.py:51-112).
@@ -65,6 +65,29 @@ __device__ __forceinline__ void epilogue_store(const GemmArgs &a, Tout *out, con
     out[row * a.ldo + col] = from_f32<Tout>(v);
 }
 
+// 8 elements at p, which need not be 16-byte aligned (one global_load_dwordx4:
+// the hardware splits what crosses a line), the first n of them valid.
+template <typename T>
+__device__ __forceinline__ u32x4 load8_any(const T *p, int64_t n) {
+    u32x4 v = {0, 0, 0, 0};
+    if (n >= 8) {
+        __builtin_memcpy(&v, p, 16);
+    } else {
+        uint16_t h[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            h[e] = 0;
+            if (e < n) __builtin_memcpy(&h[e], p + e, 2);
+        }
+        __builtin_memcpy(&v, h, 16);
+    }
+    return v;
+}
+
+// Operands of any stride and alignment, any K and N (an eager attention's
+// probabilities have rows as long as the prompt), 64-bit addresses.  It took
+// over from a SIMT kernel: bmm 32 x 777x777x128 bf16 183 -> 27 us.  What
+// bounds it: each stage waits for its loads, one stage ahead in registers.
 template <typename T, int BM, int BN, int WM, int WN, bool BCOL, typename Tout, bool SPLIT>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
     constexpr int NT = WM * WN * 64;
@@ -107,7 +130,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
             const int c = tid + i * NT, r = c >> 3, kc = c & 7;
             const int64_t gm = m0 + r, gk = k0 + kc * 8;
             if (gm < a.M && gk < kend)
-                ra[i] = *reinterpret_cast<const u32x4 *>(A + gm * a.lda + gk);
+                ra[i] = load8_any(A + gm * a.lda + gk, kend - gk);
             else
                 ra[i] = u32x4{0, 0, 0, 0};
         }
@@ -117,7 +140,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
                 const int c = tid + i * NT, r = c >> 3, kc = c & 7;
                 const int64_t gn = n0 + r, gk = k0 + kc * 8;
                 if (gn < a.N && gk < kend)
-                    rb[i] = *reinterpret_cast<const u32x4 *>(B + gn * a.ldb + gk);
+                    rb[i] = load8_any(B + gn * a.ldb + gk, kend - gk);
                 else
                     rb[i] = u32x4{0, 0, 0, 0};
             }
@@ -131,7 +154,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
                 for (int r = 0; r < 4; ++r) {
                     const int64_t gk = k0 + kb4 * 4 + r;
                     if (gn < a.N && gk < kend)
-                        rb[i * 4 + r] = *reinterpret_cast<const u32x4 *>(B + gk * a.ldb + gn);
+                        rb[i * 4 + r] = load8_any(B + gk * a.ldb + gn, a.N - gn);
                     else
                         rb[i * 4 + r] = u32x4{0, 0, 0, 0};
                 }
@@ -1229,7 +1252,7 @@ static bool dma_eligible(const GemmArgs &a, int64_t batch, bool bcol) {
 }
 
 template <typename T, typename Tout>
-static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *ws, size_t ws_bytes,
+static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int splits_req, void *ws, size_t ws_bytes,
                     hipStream_t st) {
     if constexpr (sizeof(Tout) == 2) {
         // short K (64 or 128), full 256x256 tiles, several tiles per CU: the
@@ -1237,7 +1260,7 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *
         // tile's loads
         const int64_t lim = (int64_t)1 << 30;
         const int64_t total = (a.M / 256) * (a.N / 256) * batch;
-        if (splits_req <= 1 && gemm_kernel_choice() != 1 && (a.K == 64 || a.K == 128) &&
+        if (aligned && splits_req <= 1 && gemm_kernel_choice() != 1 && (a.K == 64 || a.K == 128) &&
             a.c_kind == KUIOPS_C_NONE && a.M % 256 == 0 && a.N % 256 == 0 && 256 * a.lda + a.K < lim &&
             (bcol ? 256 * a.ldb + a.K : a.K * a.ldb + 256) < lim && a.lda % 8 == 0 && a.ldb % 8 == 0 && a.stride_a % 8 == 0 && a.stride_b % 8 == 0 && a.ldo % 8 == 0 &&
             a.stride_o % 8 == 0 && aligned16(a.out) && total >= 2 * (int64_t)num_cus() && total < INT32_MAX) {
@@ -1256,9 +1279,12 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *
     // splits_req = 0 leaves the split count to choose_tile, as far as the
     // workspace goes that max_splits asks for.
     const bool ws_ok = ws && aligned16(ws);
-    const int max_s = batch == 1 ? max_splits(a.M, a.N, a.K) : 1;
+    int max_s = batch == 1 ? max_splits(a.M, a.N, a.K) : 1;
     const size_t part = (size_t)a.M * a.N * sizeof(float);
-    if (splits_req == 0 && max_s > 1 && (!ws || ws_bytes < (size_t)max_s * part)) return KUIOPS_E_WORKSPACE;
+    if (splits_req == 0 && max_s > 1 && (!ws || ws_bytes < (size_t)max_s * part)) {
+        if (aligned) return KUIOPS_E_WORKSPACE;
+        max_s = 1;                  // (unaligned operands need no workspace)
+    }
     const TileChoice tc = choose_tile(a.M, a.N, a.K, batch, ws_ok ? max_s : 1,
                                       batch == 1 ? splits_req : 1);
     // The 256x256 tiles run 1.45 us per 64 k and about 5 us around them, one
@@ -1267,7 +1293,7 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *
     // more they win (4096^3: 98 against 122 us).
     const int64_t tiles256 = cdiv(a.M, 256) * cdiv(a.N, 256) * batch;
     const float us256 = 2.2f + (float)cdiv(tiles256, num_cus()) * ((float)(a.K / 64) * 1.45f + 3.f);
-    if (splits_req <= 1 && dma_eligible(a, batch, bcol) && (gemm_kernel_choice() == 1 || a.K < 512 || us256 <= tc.us)) {
+    if (aligned && splits_req <= 1 && dma_eligible(a, batch, bcol) && (gemm_kernel_choice() == 1 || a.K < 512 || us256 <= tc.us)) {
         a.tiles_m = (int)cdiv(a.M, 256);
         a.tiles_n = (int)cdiv(a.N, 256);
         const int vec = sizeof(Tout) == 2 ? 8 : 4;    // elements per vector store
@@ -1296,7 +1322,7 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, int splits_req, void *
         }
         return launch_status();
     }
-    const bool tile_ok = a.K > 0 && offsets_fit(a, bcol);
+    const bool tile_ok = aligned && a.K > 0 && offsets_fit(a, bcol);
     const int bk = tile_ok ? kTiles[tc.tile].bk : 64, bm = tile_ok ? kTiles[tc.tile].bm : 128,
               bn = tile_ok ? kTiles[tc.tile].bn : 128;
     int splits = tile_ok ? tc.splits : (splits_req > 0 ? splits_req : max_s);
@@ -1336,13 +1362,12 @@ static int run_simt(const GemmArgs &a, int64_t batch, bool bcol, hipStream_t st)
     return launch_status();
 }
 
-static bool mfma_eligible(const GemmArgs &a, int in_dt, bool bcol, int64_t batch) {
-    if (in_dt != KUIOPS_BF16 && in_dt != KUIOPS_F16) return false;
+// Rows of 16-byte aligned chunks, K (and a row-major B's N) multiples of 8:
+// the DMA kernels' operands.
+static bool rows_aligned(const GemmArgs &a, bool bcol, int64_t batch) {
     if (a.K % 8 || a.lda % 8 || !aligned16(a.A) || !aligned16(a.B) || a.ldb % 8) return false;
     if (batch > 1 && (a.stride_a % 8 || a.stride_b % 8)) return false;
-    if (!bcol && a.N % 8) return false;
-    if (a.M > INT32_MAX / 2 || a.N > INT32_MAX / 2) return false;
-    return true;
+    return bcol || a.N % 8 == 0;
 }
 
 // Shared entry for mm / addmm / bmm.
@@ -1356,20 +1381,18 @@ static int gemm_entry(GemmArgs a, int64_t batch, int in_dt, int out_dt, int b_la
     const bool bcol = b_layout == KUIOPS_B_COL;
     hipStream_t st = as_stream(stream);
     if (batch > 65535) return KUIOPS_E_UNSUPPORTED;
-    if (mfma_eligible(a, in_dt, bcol, batch)) {
-        if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_BF16) return run_mfma<bf16_t, bf16_t>(a, batch, bcol, splits, ws, ws_bytes, st);
-        if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_F32) return run_mfma<bf16_t, float>(a, batch, bcol, splits, ws, ws_bytes, st);
-        if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F16) return run_mfma<f16_t, f16_t>(a, batch, bcol, splits, ws, ws_bytes, st);
-        if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F32) return run_mfma<f16_t, float>(a, batch, bcol, splits, ws, ws_bytes, st);
+    if (in_dt == KUIOPS_BF16 || in_dt == KUIOPS_F16) {
+        if (a.M > INT32_MAX / 2 || a.N > INT32_MAX / 2) return KUIOPS_E_UNSUPPORTED;
+        const bool al = rows_aligned(a, bcol, batch);
+        if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_BF16) return run_mfma<bf16_t, bf16_t>(a, batch, bcol, al, splits, ws, ws_bytes, st);
+        if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_F32) return run_mfma<bf16_t, float>(a, batch, bcol, al, splits, ws, ws_bytes, st);
+        if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F16) return run_mfma<f16_t, f16_t>(a, batch, bcol, al, splits, ws, ws_bytes, st);
+        if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F32) return run_mfma<f16_t, float>(a, batch, bcol, al, splits, ws, ws_bytes, st);
         return KUIOPS_E_UNSUPPORTED;
     }
     if (cdiv(a.M, 64) > 65535 * 32 || cdiv(a.N, 64) > 65535) return KUIOPS_E_UNSUPPORTED;
     if (in_dt == KUIOPS_F32 && out_dt == KUIOPS_F32) return run_simt<float, float, float>(a, batch, bcol, st);
     if (in_dt == KUIOPS_F64 && out_dt == KUIOPS_F64) return run_simt<double, double, double>(a, batch, bcol, st);
-    if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_BF16) return run_simt<bf16_t, float, bf16_t>(a, batch, bcol, st);
-    if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_F32) return run_simt<bf16_t, float, float>(a, batch, bcol, st);
-    if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F16) return run_simt<f16_t, float, f16_t>(a, batch, bcol, st);
-    if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F32) return run_simt<f16_t, float, float>(a, batch, bcol, st);
     return KUIOPS_E_UNSUPPORTED;
 }
 

@@ -163,6 +163,25 @@ def test_addmm_tile_kernel_edges(cuda, layout, M, N, K):
     np.testing.assert_allclose(npy(o32), ref, rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,M,K,N", [(5, 77, 77, 64), (3, 130, 201, 131), (2, 1, 7, 9), (4, 333, 129, 128), (1, 257, 1031, 255)])
+@pytest.mark.parametrize("layout", ["row", "col"])
+def test_bmm_odd_strides(cuda, dtype, b, M, K, N, layout):
+    """Rows of odd length at 2-byte alignment: slices of wider NaN-filled
+    storage, so that anything read past K or N shows.  |error| <= half an ulp
+    plus fp32 sums of up to 1031 products (1e-4), inside the file's 1e-2."""
+    A, B = gen((b, M, K), dtype, seed=61), gen((b, K, N), dtype, 0.1, seed=62)
+    Aw = torch.full((b, M + 1, K + 3), float("nan"), dtype=dtype, device=cuda)
+    Ad = Aw[:, 1:, 1:K + 1].copy_(A.to(cuda))
+    shape = (b, K + 1, N + 2) if layout == "row" else (b, N + 1, K + 2)
+    Bw = torch.full(shape, float("nan"), dtype=dtype, device=cuda)
+    Bd = Bw[:, 1:, 1:-1] if layout == "row" else Bw[:, 1:, 1:-1].transpose(1, 2)
+    Bd.copy_(B.to(cuda))
+    assert_tol(ops.bmm(Ad, Bd), O.bmm(npy(A), npy(B)), dtype)
+    bias = gen((N,), dtype, seed=63)
+    assert_tol(ops.addmm(bias.to(cuda), Ad[0], Bd[0], gemv_max_m=0), O.addmm(npy(bias), npy(A[0]), npy(B[0])), dtype)
+
+
 def test_mm_rows_past_buffer_offsets(cuda):
     """A row-major B whose rows lie 32 MiB apart (offsets past 2^31 bytes)."""
     M, N, K, ld = 130, 64, 72, 1 << 24
