@@ -24,8 +24,8 @@
 // same XCD (dispatch is round-robin over the 8 XCDs, each with its own L2)
 // and are visited in groups of 8 tile-rows.
 //
-// f32 / f64 operands take `gemm_simt_kernel`, a plain LDS-tiled kernel with
-// the same epilogue.
+// f32: `gemm_f32_kernel`, fp32 MFMAs.  f64: `gemm_simt_kernel`, a plain
+// LDS-tiled kernel with the same epilogue.
 //
 // Semantics follow aten mm / addmm / bmm (the reference's fallthrough and
 // test oracle, kuipy/kuiops.py:403-564, tests/test_jit_ops.py:51-112).
@@ -1077,8 +1077,140 @@ void gemm_wave_kernel(GemmArgs a) {
     }
 }
 
-// Generic LDS-tiled SIMT GEMM (any strides / shapes / float dtypes): 64x64
-// tile, 256 threads each owning a 4x4 strided patch, K step 16.
+// ------------------------------------------------------------------------
+// gemm_f32_kernel: fp32 GEMM on 32x32x2 fp32 MFMAs (fp32 products and sums),
+// any strides, sizes and alignments.  WM x WN waves of 32x32 output tiles, WK
+// K slices per stage of 32 k each (a slice's waves compute it alone; slices
+// are summed in order at the end).
+//   * MFMA sums over k in any order, so a lane of half h takes k 4h .. 4h + 3
+//     of each 8: A (and a K-contiguous B) is one ds_read_b128 per 4 MFMAs from
+//     rows of 36 floats (16 consecutive rows on distinct 16-byte slots); a
+//     row-major B stays [k][n], read by ds_read_b32 from rows of BN + 8 floats
+//     (the two halves' rows on the two halves of the 64 banks).
+//   * The next stage's loads are in flight in registers under a stage's MFMAs.
+// What bounds it: large sizes the fp32 MFMAs (4096^3 1.23 ms, 112 of 157
+// TFLOP/s; the SIMT kernel that ran here before 2.61 ms), small ones the load
+// of a stage, one ahead (64 x 3072 x 768: 192 work-groups of 32x32 tiles 10.9
+// us, against 152 for 48 SIMT ones).
+template <typename F>
+__device__ __forceinline__ f32x4 load4_any(const F *p, int64_t n) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (n >= 4) {
+        __builtin_memcpy(&v, p, 16);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (e < n) v[e] = p[e];
+    }
+    return v;
+}
+
+template <int WM, int WN, int WK, bool BCOL>
+__global__ __launch_bounds__(WM * WN * WK * 64) void gemm_f32_kernel(GemmArgs a) {
+    constexpr int NT = WM * WN * WK * 64, BM = WM * 32, BN = WN * 32, BK = 32 * WK;
+    constexpr int PA = 36, PB = BN + 8;                        // LDS row pitches (floats)
+    constexpr int CA = BM * BK / 4 / NT, CB = BN * BK / 4 / NT;    // 16-byte chunks per thread
+    static_assert(CA >= 1 && CB >= 1, "tile / thread mismatch");
+    constexpr int ASL = BM * PA, BSL = BCOL ? BN * PA : 32 * PB;   // floats per K slice
+    __shared__ __attribute__((aligned(16))) float sA[2][WK * ASL], sB[2][WK * BSL];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+    const int lr = lane & 31, h = lane >> 5;
+    int tm, tn, bz;
+    tile_coords_batched(blockIdx.x, gridDim.x, a.tiles_m, a.tiles_n, tm, tn, bz);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+    const float *A = reinterpret_cast<const float *>(a.A) + bz * a.stride_a;
+    const float *B = reinterpret_cast<const float *>(a.B) + bz * a.stride_b;
+
+    f32x4 ra[CA], rb[CB];
+    auto load = [&](int64_t k0) {
+#pragma unroll
+        for (int i = 0; i < CA; ++i) {
+            const int c = tid + i * NT, r = c / (BK / 4);
+            const int64_t gm = m0 + r, gk = k0 + c % (BK / 4) * 4;
+            ra[i] = load4_any(A + gm * a.lda + gk, gm < a.M ? a.K - gk : 0);
+        }
+#pragma unroll
+        for (int i = 0; i < CB; ++i) {
+            const int c = tid + i * NT;
+            if constexpr (BCOL) {
+                const int64_t gn = n0 + c / (BK / 4), gk = k0 + c % (BK / 4) * 4;
+                rb[i] = load4_any(B + gn * a.ldb + gk, gn < a.N ? a.K - gk : 0);
+            } else {
+                const int64_t gk = k0 + c / (BN / 4), gn = n0 + c % (BN / 4) * 4;
+                rb[i] = load4_any(B + gk * a.ldb + gn, gk < a.K ? a.N - gn : 0);
+            }
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < CA; ++i) {
+            const int c = tid + i * NT, r = c / (BK / 4), kc = c % (BK / 4);
+            *reinterpret_cast<f32x4 *>(&sA[buf][(kc >> 3) * ASL + r * PA + (kc & 7) * 4]) = ra[i];
+        }
+#pragma unroll
+        for (int i = 0; i < CB; ++i) {
+            const int c = tid + i * NT;
+            if constexpr (BCOL) {
+                const int r = c / (BK / 4), kc = c % (BK / 4);
+                *reinterpret_cast<f32x4 *>(&sB[buf][(kc >> 3) * BSL + r * PA + (kc & 7) * 4]) = rb[i];
+            } else {
+                const int k = c / (BN / 4), nc = c % (BN / 4);
+                *reinterpret_cast<f32x4 *>(&sB[buf][(k >> 5) * BSL + (k & 31) * PB + nc * 4]) = rb[i];
+            }
+        }
+    };
+
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    const int nk = (int)((a.K + BK - 1) / BK);
+    if (nk > 0) {
+        load(0);
+        store(0);
+    }
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+        const int buf = kt & 1;
+        if (kt + 1 < nk) load((int64_t)(kt + 1) * BK);
+        const float *pa = sA[buf] + wk * ASL + (wm * 32 + lr) * PA + 4 * h;
+        const float *pb = sB[buf] + wk * BSL + (BCOL ? (wn * 32 + lr) * PA + 4 * h : 4 * h * PB + wn * 32 + lr);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const f32x4 fa = *reinterpret_cast<const f32x4 *>(pa + 8 * g);
+            f32x4 fb;
+            if constexpr (BCOL) {
+                fb = *reinterpret_cast<const f32x4 *>(pb + 8 * g);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) fb[t] = pb[(8 * g + t) * PB];
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[t], fb[t], acc, 0, 0, 0);
+        }
+        if (kt + 1 < nk) store(buf ^ 1);
+        __syncthreads();
+    }
+    if constexpr (WK > 1) {
+        // K slices summed in slice order by the first slice's waves
+        float *red = sA[0];
+        static_assert((WK - 1) * WM * WN * 1024 <= 2 * WK * ASL, "slice sums fit");
+        if (wk > 0) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) red[((wave - WM * WN) * 16 + e) * 64 + lane] = acc[e];
+        }
+        __syncthreads();
+        if (wk > 0) return;
+#pragma unroll
+        for (int z = 1; z < WK; ++z)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] += red[(((z - 1) * WM * WN + wave) * 16 + e) * 64 + lane];
+    }
+    a.out = reinterpret_cast<float *>(a.out) + bz * a.stride_o;
+    store_tile32<float>(a, acc, m0 + wm * 32, n0 + wn * 32 + lr, h);
+}
+
+// LDS-tiled SIMT GEMM (fp64; any strides and shapes): 64x64 tile, 256 threads each owning a 4x4 strided patch, K step 16.
 template <typename Tin, typename Tacc, typename Tout>
 __global__ __launch_bounds__(256) void gemm_simt_kernel(GemmArgs a, int b_col) {
     __shared__ Tacc sA[16][65];
@@ -1355,6 +1487,26 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
     return launch_status();
 }
 
+// 64x64 tiles where they give every CU a work-group, else 32x32 (us, 64x64
+// against 32x32: 512 x 2048 x 2048 58 / 61, 2048^3 175 / 228, 200 x 3000 x 1003
+// 42 / 31, 19 x 16256 x 5056 184 / 83), whose K is split over 8 waves instead
+// of 4 while one work-group per CU runs (1 x 4096 x 4096 48 -> 41).
+static int run_f32(GemmArgs a, int64_t batch, bool bcol, hipStream_t st) {
+    const bool big = a.M > 32 && cdiv(a.M, 64) * cdiv(a.N, 64) * batch >= num_cus();
+    const int64_t tm = cdiv(a.M, big ? 64 : 32), tn = cdiv(a.N, big ? 64 : 32);
+    if (tm * tn * batch > INT32_MAX) return KUIOPS_E_UNSUPPORTED;
+    a.tiles_m = (int)tm;
+    a.tiles_n = (int)tn;
+    const dim3 grid((unsigned)(tm * tn * batch)), block(256);
+    if (big && bcol) hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 1, true>), grid, block, 0, st, a);
+    else if (big) hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 1, false>), grid, block, 0, st, a);
+    else if (tm * tn * batch <= num_cus() && bcol) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 8, true>), grid, dim3(512), 0, st, a);
+    else if (tm * tn * batch <= num_cus()) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 8, false>), grid, dim3(512), 0, st, a);
+    else if (bcol) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 4, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 4, false>), grid, block, 0, st, a);
+    return launch_status();
+}
+
 template <typename Tin, typename Tacc, typename Tout>
 static int run_simt(const GemmArgs &a, int64_t batch, bool bcol, hipStream_t st) {
     dim3 grid((unsigned)cdiv(a.M, 64), (unsigned)cdiv(a.N, 64), (unsigned)batch);
@@ -1391,7 +1543,7 @@ static int gemm_entry(GemmArgs a, int64_t batch, int in_dt, int out_dt, int b_la
         return KUIOPS_E_UNSUPPORTED;
     }
     if (cdiv(a.M, 64) > 65535 * 32 || cdiv(a.N, 64) > 65535) return KUIOPS_E_UNSUPPORTED;
-    if (in_dt == KUIOPS_F32 && out_dt == KUIOPS_F32) return run_simt<float, float, float>(a, batch, bcol, st);
+    if (in_dt == KUIOPS_F32 && out_dt == KUIOPS_F32) return run_f32(a, batch, bcol, st);
     if (in_dt == KUIOPS_F64 && out_dt == KUIOPS_F64) return run_simt<double, double, double>(a, batch, bcol, st);
     return KUIOPS_E_UNSUPPORTED;
 }

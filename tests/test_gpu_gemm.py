@@ -182,6 +182,32 @@ def test_bmm_odd_strides(cuda, dtype, b, M, K, N, layout):
     assert_tol(ops.addmm(bias.to(cuda), Ad[0], Bd[0], gemv_max_m=0), O.addmm(npy(bias), npy(A[0]), npy(B[0])), dtype)
 
 
+@pytest.mark.parametrize("layout", ["row", "col"])
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 96), (33, 31, 257), (64, 3072, 768), (300, 1000, 1003), (1000, 1030, 130), (7, 9000, 5)])
+def test_mm_f32_tiles(cuda, layout, M, N, K):
+    """fp32 MFMA tiles (32x32 with 8 and 4 K slices, 64x64), ragged in every
+    size, operands inside NaN-filled storage, against a 64-bit product:
+    fp32 sums of K products of size s are within K * 2^-24 * sum|s|, here
+    taken as the root-mean-square bound 2^-24 * K relative to the row norms."""
+    A, B = gen((M, K), torch.float32, seed=71), gen((K, N), torch.float32, 0.1, seed=72)
+    Ad = torch.full((M + 1, K + 5), float("nan"), device=cuda)[1:, 3:K + 3].copy_(A.to(cuda))
+    Bw = torch.full((K + 1, N + 2) if layout == "row" else (N + 1, K + 2), float("nan"), device=cuda)
+    Bd = Bw[1:, 1:-1] if layout == "row" else Bw[1:, 1:-1].t()
+    Bd.copy_(B.to(cuda))
+    ref = A.double() @ B.double()
+    bound = K * 2.0 ** -24 * (A.double().norm(dim=1, keepdim=True) * B.double().norm(dim=0, keepdim=True))
+    out = ops.mm(Ad, Bd)
+    assert ((out.cpu().double() - ref).abs() <= bound).all()
+    bias, C = gen((N,), torch.float32, seed=73), gen((M, N), torch.float32, seed=74)
+    got = ops.addmm(bias.to(cuda), Ad, Bd)
+    assert ((got.cpu().double() - ref - bias.double()).abs() <= bound + 1e-5).all()
+    got = ops.addmm(C.to(cuda), Ad, Bd, beta=2.0, alpha=0.5)
+    assert ((got.cpu().double() - 0.5 * ref - 2 * C.double()).abs() <= bound + 1e-5).all()
+    batch = ops.bmm(Ad.expand(3, -1, -1), Bd.expand(3, -1, -1))
+    # (a batch has more tiles, so its K may be sliced otherwise)
+    assert ((batch[2].cpu().double() - ref).abs() <= bound).all()
+
+
 def test_mm_rows_past_buffer_offsets(cuda):
     """A row-major B whose rows lie 32 MiB apart (offsets past 2^31 bytes)."""
     M, N, K, ld = 130, 64, 72, 1 << 24
