@@ -458,6 +458,193 @@ __global__ __launch_bounds__(128) void fa_decode_combine_kernel(AttnArgs a) {
     if (a.lse && tid == 0) a.lse[grow] = L > 0.f ? (M + __log2f(L)) * kLn2 : -INFINITY;
 }
 
+// fa_decode_mfma_kernel: split-KV decode for 3 or more query rows per KV head
+// (up to 16 per work-group; grouped-query attention), on 16x16x32 MFMAs.  A
+// wave takes steps of 32 keys of the split by itself:
+//   * S^T = K Q^T: K goes from memory straight into the A operand (lane: one
+//     key, 16 bytes of its row per MFMA); a lane of the result holds 8 keys of
+//     one query row, so a probability is computed once (the VALU form computes
+//     it in every lane of a key's group).
+//   * O^T += V^T P^T: V goes to LDS by DMA and is read transposed
+//     (ds_read_b64_tr_b16; keys numbered in the order the score accumulator
+//     holds them).  P stays exact to fp32 rounding of the result: it is the
+//     sum of two 16-bit halves (P = hi + lo, 2^-17 relative for bf16), one MFMA each.
+// K and V descriptors end at the sequence's key count (device memory), so keys
+// past it are neither fetched nor seen, and its keys are spread evenly over
+// the splits.  What bounds it: the K / V stream (16 sequences of 2000-4000
+// keys, GQA 32/8, head dim 128: 57 us for the VALU form, which also read the
+// caches to their capacity, 44.5 now).
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void fa_decode_mfma_kernel(AttnArgs a) {
+    constexpr int NWV = 4, KB = 32, R = 16;
+    constexpr int RB = HD * 2, VT = KB * RB;          // bytes per V row / wave tile
+    constexpr int KK = HD / 32, DT = HD / 16, DV = VT / 1024;
+    typedef typename Mfma<T>::frag frag;
+    typedef T t2v __attribute__((ext_vector_type(2)));
+    // two V tiles per wave
+    __shared__ __attribute__((aligned(1024))) char sV0[NWV * VT], sV1[NWV * VT];
+    __shared__ float sm[NWV][R], sl[NWV][R];
+    static_assert(R * HD * 4 == VT, "a wave's state takes its V tile");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, G4 = lane >> 4;
+    int unit = blockIdx.y;
+    if (gridDim.x == 1 && (gridDim.y & 7) == 0) unit = (unit & 7) * (gridDim.y >> 3) + (unit >> 3);
+    const int split = blockIdx.x;
+    const int64_t b = blockIdx.z;
+    const int hk = unit / a.row_groups, rg = unit % a.row_groups;
+    const int G = (int)a.hq / (int)a.hkv, LQ = (int)a.l, rows_kv = G * LQ;
+    const int r0 = rg * a.rows_per_group;
+
+    const int s_b = (int)(a.kv_len ? max((int64_t)0, min((int64_t)a.kv_len[b], a.s)) : a.s);
+    const int chunk = (int)min(a.chunk, (int64_t)((s_b + a.splits * KB - 1) / (a.splits * KB)) * KB);
+    const int kbeg = split * chunk, kend = min(s_b, kbeg + chunk);
+
+    const T *Kp = reinterpret_cast<const T *>(a.K) + b * a.sk0 + hk * a.sk1;
+    const T *Vp = reinterpret_cast<const T *>(a.V) + b * a.sv0 + hk * a.sv1;
+    const uint32_t kbytes = kend > 0 ? (uint32_t)(((int64_t)(kend - 1) * a.sk2 + HD) * 2) : 0u;
+    const uint32_t vbytes = kend > 0 ? (uint32_t)(((int64_t)(kend - 1) * a.sv2 + HD) * 2) : 0u;
+    const __amdgpu_buffer_rsrc_t rsK = make_rsrc(Kp, kbytes), rsV = make_rsrc(Vp, vbytes);
+
+    // this lane's query row: row r0 + lr (B operand; rows past the group are 0)
+    const int rr = r0 + lr;
+    const bool row_ok = lr < a.rows_per_group && rr < rows_kv;
+    const int64_t qhead = hk * G + (row_ok ? rr / LQ : 0), qi = row_ok ? rr % LQ : 0;
+    frag qf[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+        qf[kk] = as_frag<frag>(row_ok ? *reinterpret_cast<const u32x4 *>(reinterpret_cast<const T *>(a.Q) + b * a.sq0 +
+                                                                       qhead * a.sq1 + qi * a.sq2 + kk * 32 + G4 * 8)
+                                      : u32x4{0, 0, 0, 0});
+    // keys visible to this row (exclusive bound)
+    const int lim = row_ok ? min(kend, (int)(a.causal ? s_b - a.l + qi + 1 : s_b)) : 0;
+
+    // V tile: 16-byte chunk c of row r at position c ^ 2 f(r): the 16 rows x 32
+    // bytes of a transposing read fall on the 64 banks evenly.
+    auto vsw = [](int r) { return HD == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); };
+    uint32_t offV[DV];
+#pragma unroll
+    for (int j = 0; j < DV; ++j) {
+        const int ch = j * 64 + lane, r = ch / (HD / 8), c = (ch % (HD / 8)) ^ vsw(r);
+        offV[j] = (uint32_t)((r * a.sv2 + c * 8) * 2);
+    }
+    const uint32_t offK = (uint32_t)((lr * a.sk2 + G4 * 8) * 2), stepK = (uint32_t)(16 * a.sk2 * 2);
+    int offVr[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        const int r = 4 * G4 + (lr >> 2), d = dt * 16 + 4 * (lr & 3);
+        offVr[dt] = r * RB + (((d >> 3) ^ vsw(r)) << 4) + ((d >> 2) & 1) * 8;      // vsw(r + 16) == vsw(r)
+    }
+    constexpr uint32_t kOut = 0x80000000u;
+    u32x4 kr[2][2][KK];
+    // keys k0 .. k0 + 31: K into slot sl, V into tile sv (nothing past kend)
+    auto issue = [&](int k0, int slot, char *sv) __attribute__((always_inline)) {
+        const bool on = k0 < kend;
+        const uint32_t kb = on ? (uint32_t)((int64_t)k0 * a.sk2 * 2) : kOut;
+        const uint32_t vb = on ? (uint32_t)((int64_t)k0 * a.sv2 * 2) : kOut;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk)
+                kr[slot][t][kk] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                    rsK, (int)(kb + offK + t * stepK + kk * 64), 0, 0));
+#pragma unroll
+        for (int j = 0; j < DV; ++j) dma16_buf(rsV, vb + offV[j], 0, sv + wave * VT + j * 1024);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    f32x4 o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_used = -INFINITY, l_run = 0.f;
+    auto step = [&](int k0, int slot, const char *sv) __attribute__((always_inline)) {
+        f32x4 sc[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            sc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) sc[t] = Mfma<T>::m16(as_frag<frag>(kr[slot][t][kk]), qf[kk], sc[t]);
+        }
+        // slot (t, i): key k0 + 16 t + 4 G4 + i
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sc[t][i] = k0 + 16 * t + 4 * G4 + i < lim ? sc[t][i] * a.scale_log2 : -INFINITY;
+                mx = fmaxf(mx, sc[t][i]);
+            }
+        mx = xor_max<32>(xor_max<16>(mx));
+        if (__any(mx > m_used + kRescaleSlack)) {
+            const float m_new = fmaxf(m_used, mx);
+            const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_used - m_new);
+            l_run *= alpha;
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[t][i] *= alpha;
+            m_used = m_new;
+        }
+        const float mref = m_used == -INFINITY ? 0.f : m_used;
+        typedef T t8 __attribute__((ext_vector_type(8)));
+        t8 hi, lo;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float p = fast_exp2(sc[t][i] - mref);
+                l_run += p;
+                hi[4 * t + i] = from_f32<T>(p);
+                lo[4 * t + i] = from_f32<T>(p - to_f32(hi[4 * t + i]));
+            }
+        const frag fh = __builtin_bit_cast(frag, hi), fl = __builtin_bit_cast(frag, lo);
+        // this step's V tile has landed: only the next step's loads are younger
+        constexpr int Y = 2 * KK + DV;
+        __builtin_amdgcn_s_waitcnt((Y & 15) | ((Y >> 4) << 14) | (7 << 4) | (15 << 8));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const char *vb = sv + wave * VT + offVr[dt];
+            const s16x4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4 *)to_lds(vb));
+            const s16x4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4 *)to_lds(vb + 16 * RB));
+            const u32x2 h0 = __builtin_bit_cast(u32x2, t0), h1 = __builtin_bit_cast(u32x2, t1);
+            const frag vf = as_frag<frag>(u32x4{h0[0], h0[1], h1[0], h1[1]});
+            o[dt] = Mfma<T>::m16(vf, fh, o[dt]);
+            o[dt] = Mfma<T>::m16(vf, fl, o[dt]);
+        }
+    };
+
+    constexpr int KS = NWV * KB;
+    int k0 = kbeg + wave * KB;
+    issue(k0, 0, sV0);
+    for (; k0 < kend; k0 += 2 * KS) {
+        issue(k0 + KS, 1, sV1);
+        step(k0, 0, sV0);
+        // (this wave's reads of the tile are done before its refill)
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_sched_barrier(0);
+        issue(k0 + 2 * KS, 0, sV0);
+        step(k0 + KS, 1, sV1);
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // the wave's state takes the place of its first V tile, once its DMA is done
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_sched_barrier(0);
+    float (*so)[R][HD] = reinterpret_cast<float (*)[R][HD]>(sV0);
+    // lanes of a row hold disjoint keys: row sums over the lane groups
+    l_run = xor_add<32>(xor_add<16>(l_run));
+    if (G4 == 0) {
+        sm[wave][lr] = m_used;
+        sl[wave][lr] = l_run;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4 *>(&so[wave][lr][dt * 16 + 4 * G4]) = o[dt];
+    decode_finish<T, HD, R, NWV, NWV * 64>(a, split, b, hk, rg, r0, sm, sl, so);
+}
+
 // ------------------------------------------------------------------------
 // sdpa_general_kernel -- every other SDPA: fp32 / fp64 (and 16-bit) inputs,
 // head dims e != ev, head dims past the MFMA kernels' 64 / 128, an optional
@@ -620,8 +807,14 @@ static int64_t decode_chunk(int64_t s) {
     return c < 64 ? 64 : c;
 }
 
-// Query rows per work-group (the rows sharing a KV head, up to 8).
-static int decode_rows_per_group(int rows_kv) {
+// Query rows per work-group (of the rows sharing a KV head): 16 on the MFMA
+// kernel, which takes 3 or more rows (with one or two its MFMAs are mostly
+// empty and the VALU form has little to do) and key rows whose byte offsets
+// fit 31 bits; else up to 8.
+constexpr int kMfmaRows = 16;
+static int decode_rows_per_group(int64_t s, int rows_kv, int64_t sk2, int64_t sv2) {
+    const int64_t st = sk2 > sv2 ? sk2 : sv2;
+    if (rows_kv >= 3 && s < (1 << 30) && sk2 >= 0 && sv2 >= 0 && (s + 64) * st * 2 < ((int64_t)1 << 31)) return kMfmaRows;
     return rows_kv <= 1 ? 1 : rows_kv <= 2 ? 2 : rows_kv <= 4 ? 4 : 8;
 }
 
@@ -652,10 +845,14 @@ static bool decode_row_wide(int64_t s, int64_t hd, int64_t rows) {
 }
 
 // Keys per split for a launch of `groups` row-group work-groups per split:
-// enough splits for about two work-groups per CU, at most 32, and never
-// fewer keys than decode_chunk (the workspace is sized by it).
-static int64_t decode_chunk_for(int64_t s, int64_t groups) {
-    const int64_t want = cdiv(2 * (int64_t)num_cus(), groups > 0 ? groups : 1);
+// enough splits for about `per_cu` work-groups per CU, at most 32, and never
+// fewer keys than decode_chunk (the workspace is sized by it).  Two per CU on
+// the VALU kernels; one on the MFMA kernel, whose waves keep two steps in
+// flight and whose states have 16 rows to merge (us, one against two: 8
+// sequences of 1024 keys 14.0 / 17.7, 16 of 4000 46.0 / 45.6, 1 of 16384 21.2 /
+// 20.9; 2 KV heads, 16 of 8000 37.5 / 47.7).
+static int64_t decode_chunk_for(int64_t s, int64_t groups, int per_cu) {
+    const int64_t want = cdiv(per_cu * (int64_t)num_cus(), groups > 0 ? groups : 1);
     const int64_t splits = want < 1 ? 1 : (want > 32 ? 32 : want);
     const int64_t c = cdiv(cdiv(s, splits), 64) * 64;
     return c < decode_chunk(s) ? decode_chunk(s) : c;
@@ -727,10 +924,18 @@ static int launch_decode(AttnArgs a, hipStream_t st) {
                            dim3(kDecodeWideWaves * 64), 0, st, a);
         return launch_status();
     }
-    const int R = decode_rows_per_group(rows_kv);
+    const int R = decode_rows_per_group(a.s, rows_kv, a.sk2, a.sv2);
     a.rows_per_group = R;
     a.row_groups = (int)cdiv(rows_kv, R);
     dim3 grid((unsigned)a.splits, (unsigned)(a.hkv * a.row_groups), (unsigned)a.n);
+    if (R == kMfmaRows) {
+        const bool fused = a.splits <= kFusedMergeMaxSplits && a.n * a.hkv * a.row_groups <= kMaxSplitGroups;
+        if (!fused) a.counters = nullptr;
+        hipLaunchKernelGGL((fa_decode_mfma_kernel<T, HD>), grid, dim3(256), 0, st, a);
+        if (!fused && a.splits > 1)
+            hipLaunchKernelGGL((fa_decode_combine_kernel<T, HD>), dim3((unsigned)(a.n * a.hq * a.l)), dim3(128), 0, st, a);
+        return launch_status();
+    }
     if (a.splits == 1) {
         // short caches: one work-group per row group streams every key (no
         // workspace round trip).  Four rows take 4-wave work-groups: at 180
@@ -832,8 +1037,8 @@ extern "C" int kuiops_sdpa_decode(int64_t n, int64_t hq, int64_t hkv, int64_t l,
     fill_args(a, n, hq, hkv, l, s, Q, sq, K, sk, V, sv, O, so, lse, scale, causal);
     a.kv_len = kv_len;
     const int64_t ss = s > 0 ? s : 1;
-    const int R = decode_rows_per_group((int)((hq / hkv) * l));
-    a.chunk = decode_chunk_for(ss, n * hkv * cdiv((hq / hkv) * l, R));
+    const int R = decode_rows_per_group(s, (int)((hq / hkv) * l), a.sk2, a.sv2);
+    a.chunk = decode_chunk_for(ss, n * hkv * cdiv((hq / hkv) * l, R), R == kMfmaRows ? 1 : 2);
     if (decode_row_wide(ss, ev, n * hq * l) || decode_single_split(ss, ev, R)) a.chunk = ss;
     a.splits = (int)cdiv(ss, a.chunk);
     const int64_t rows = n * hq * l;

@@ -68,6 +68,159 @@ __device__ __forceinline__ void merge_state(float &m1, float &l1, float *o1, flo
     m1 = M;
 }
 
+// 4 output values v * scale (8-byte aligned: output strides are multiples of 4).
+template <typename T>
+__device__ __forceinline__ void decode_store4(T *p, f32x4 v, float scale) {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    t4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = from_f32<T>(v[e] * scale);
+    *reinterpret_cast<t4 *>(p) = w;
+}
+
+// The wave states of a work-group (slot w: maximum sm[w][r], sum sl[w][r],
+// unnormalised output so[w][r][d] of row r0 + r), merged in slot order: a
+// single split writes the normalised output; otherwise the split's state goes
+// to the workspace and, with arrival counters, the last split work-group of
+// the row group merges the splits.
+template <typename T, int HD, int R, int NSL, int NT>
+__device__ __forceinline__ void decode_finish(const AttnArgs &a, int split, int64_t b, int hk, int rg, int r0,
+                                              const float (*sm)[R], const float (*sl)[R],
+                                              const float (*so)[R][HD]) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NWV = NT / 64;
+    const int G = (int)a.hq / (int)a.hkv, LQ = (int)a.l, rows_kv = G * LQ;
+    __syncthreads();
+    const int nrows = min(a.rows_per_group, rows_kv - r0);
+    constexpr int D4 = HD / 4;                 // a thread takes 4 adjacent output columns
+    // agent-coherent (sc1) accesses of the split states, written through the
+    // XCD's L2 and read past it: the work-group that merges the splits may run
+    // on another XCD
+    constexpr int kSc1 = kSc1Aux;
+    const __amdgpu_buffer_rsrc_t rs_ml = __builtin_amdgcn_make_buffer_rsrc((void *)a.ws_ml, (short)0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs_o = __builtin_amdgcn_make_buffer_rsrc((void *)a.ws_o, (short)0, 0x7fffffff, 0x00020000);
+    for (int idx = tid; idx < nrows * D4; idx += NT) {
+        const int r = idx / D4, d = idx % D4 * 4;
+        // max over the slots, then one weight per slot for its sum and output
+        // (independent terms, summed in slot order)
+        float mm = -INFINITY;
+        for (int sv = 0; sv < NSL; ++sv) mm = fmaxf(mm, sm[sv][r]);
+        const float mu = (mm == -INFINITY) ? 0.f : mm;
+        float ll = 0.f;
+        f32x4 oo = {0.f, 0.f, 0.f, 0.f};
+        for (int sv = 0; sv < NSL; ++sv) {
+            const float wgt = fast_exp2(sm[sv][r] - mu);
+            ll = __builtin_fmaf(sl[sv][r], wgt, ll);
+            const f32x4 ov = *reinterpret_cast<const f32x4 *>(&so[sv][r][d]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oo[e] = __builtin_fmaf(ov[e], wgt, oo[e]);
+        }
+        const int rr = r0 + r;
+        const int64_t head = hk * G + rr / LQ, qi = rr % LQ;
+        const int64_t grow = (b * a.hq + head) * a.l + qi;
+        if (a.splits == 1) {
+            const float inv = ll > 0.f ? 1.f / ll : 0.f;
+            decode_store4<T>(reinterpret_cast<T *>(a.O) + b * a.so0 + head * a.so1 + qi * a.so2 + d, oo, inv);
+            if (a.lse && d == 0) a.lse[grow] = ll > 0.f ? (mm + __log2f(ll)) * kLn2 : -INFINITY;
+            continue;
+        }
+        const int64_t st = grow * a.splits + split;
+        if (!a.counters) {
+            // merged by the separate merge kernel
+            *reinterpret_cast<f32x4 *>(&a.ws_o[st * HD + d]) = oo;
+            if (d == 0) {
+                a.ws_ml[st * 2 + 0] = mm;
+                a.ws_ml[st * 2 + 1] = ll;
+            }
+            continue;
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, oo), rs_o, (int)((st * HD + d) * 4), 0, kSc1);
+        if (d == 0)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, f32x2{mm, ll}), rs_ml, (int)(st * 8), 0, kSc1);
+    }
+    if (a.splits == 1 || !a.counters) return;
+
+    // The last of the group's split work-groups to arrive merges the splits
+    // in split order (bitwise repeatable whatever the arrival order).
+    // Ordering (as in the decode GEMM's merge): the split states are sc1
+    // stores (what an agent-scope relaxed atomic store is, written through
+    // the per-XCD L2); each thread waits for their acknowledgements
+    // (s_waitcnt(0)) before the barrier that precedes tid 0's agent-scope
+    // counter RMW, and the merging work-group reads them with sc1 buffer
+    // loads, which miss the non-coherent caches.  This relies on the hardware
+    // rule that an acknowledged sc1 store is visible at the agent's coherence
+    // point before a later RMW of the same agent, not on a release / acquire
+    // pair (which would add an L2 write-back per XCD to every work-group).
+    __shared__ int s_last;
+    __shared__ float s_w[R][64];
+    __shared__ float s_M[R], s_L[R];
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    unsigned *ctr = a.counters + ((b * a.hkv + hk) * a.row_groups + rg) * kAttnCounterStride;
+    if (tid == 0)
+        s_last = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 (unsigned)(a.splits - 1);
+    __syncthreads();
+    if (!s_last) return;
+    // The split states are read with agent-coherent (sc1) buffer loads, which
+    // unlike atomics can be batched.  Wave w turns row w's split maxima into
+    // weights (splits <= 64, one per lane); a thread then sums weight *
+    // o[split] over its 4 columns in split order.
+    auto grow_of = [&](int r) {
+        const int rr = r0 + r;
+        return (b * a.hq + hk * G + rr / LQ) * a.l + rr % LQ;
+    };
+    // A thread's o loads go out together (16 rows of 8 splits, one column a
+    // thread and 8 loads at a time, took 8 round trips), the first ones before
+    // the weights are known.
+    constexpr int kMaxSplits = 16;             // (more are merged by the separate kernel)
+    f32x4 ov[kMaxSplits];
+    auto load_o = [&](int idx) __attribute__((always_inline)) {
+        const uint32_t base = (uint32_t)((grow_of(idx / D4) * a.splits * HD + idx % D4 * 4) * 4);
+#pragma unroll
+        for (int z = 0; z < kMaxSplits; ++z)
+            if (z < a.splits)
+                ov[z] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      rs_o, (int)(base + (uint32_t)(z * HD * 4)), 0, kSc1));
+    };
+    if (tid < nrows * D4) load_o(tid);
+    for (int r = wave; r < nrows; r += NWV) {
+        const uint32_t base = (uint32_t)(grow_of(r) * a.splits * 2) * 4;
+        // (the b32 loads return raw bits)
+        const float mz = lane < a.splits
+                             ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_ml, base + lane * 8, 0, kSc1))
+                             : -INFINITY;
+        const float lz = lane < a.splits
+                             ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_ml, base + lane * 8 + 4, 0, kSc1))
+                             : 0.f;
+        const float M = wave_max(mz);
+        const float Mu = (M == -INFINITY) ? 0.f : M;
+        const float w = lane < a.splits ? fast_exp2(mz - Mu) : 0.f;
+        s_w[r][lane] = w;
+        const float L = wave_sum(w * lz);
+        if (lane == 0) { s_M[r] = M; s_L[r] = L; }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < nrows * D4; idx += NT) {
+        const int r = idx / D4, d = idx % D4 * 4;
+        if (idx != tid) load_o(idx);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int z = 0; z < kMaxSplits; ++z)
+            if (z < a.splits) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += s_w[r][z] * ov[z][e];
+            }
+        const float L = s_L[r];
+        const int rr = r0 + r;
+        const int64_t head = hk * G + rr / LQ, qi = rr % LQ;
+        decode_store4<T>(reinterpret_cast<T *>(a.O) + b * a.so0 + head * a.so1 + qi * a.so2 + d, acc, L > 0.f ? 1.f / L : 0.f);
+        if (a.lse && d == 0) a.lse[grow_of(r)] = L > 0.f ? (s_M[r] + __log2f(L)) * kLn2 : -INFINITY;
+    }
+    if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // One work-group of fa_decode_kernel: split `split` of the row group `unit`
 // (KV head * row_groups + row group) of batch entry b.  The query is read
 // first, then every step loads its keys.
@@ -107,9 +260,11 @@ __device__ __forceinline__ void fa_decode_block(const AttnArgs &a, int split, in
         for (int e = 0; e < 8; ++e) o[r][e] = 0.f;
     }
 
-    // The loop runs over the split's keys within the capacity s (known at
-    // launch), not over the device key count: the K / V loads then need not
-    // wait for kv_len.  Keys at or past kend are masked after loading.
+    // The first step's addresses are bounded by the capacity s (known at
+    // launch), not by the device key count, so its K / V loads need not wait
+    // for kv_len; keys at or past kend are masked after loading.  Later steps
+    // stop at kend (24 sequences of 750-1500 keys, 32 heads of 128: 104 ->
+    // 81 us).
     const int64_t kend_cap = min(a.s, kbeg + a.chunk);
     u32x4 kr[NB], vr[NB];
     auto load_kv = [&](int64_t kb) __attribute__((always_inline)) {
@@ -158,7 +313,7 @@ __device__ __forceinline__ void fa_decode_block(const AttnArgs &a, int split, in
         last_key[r] = ok ? (a.causal ? s_b - a.l + qi + 1 : s_b) : 0;
     }
 
-    for (int64_t kb = kb0; kb < kend_cap; kb += kstep) {
+    for (int64_t kb = kb0; kb < kend; kb += kstep) {
         float s[R][NB];
         if constexpr (!KVFIRST) load_kv(kb);
         // keys past the device count are zeroed (their scores are masked
@@ -217,7 +372,7 @@ __device__ __forceinline__ void fa_decode_block(const AttnArgs &a, int split, in
             }
         }
         if constexpr (KVFIRST)
-            if (kb + kstep < kend_cap) load_kv(kb + kstep);
+            if (kb + kstep < kend) load_kv(kb + kstep);
     }
 
     // Merge the KPW key slots of a wave (lanes with equal dl) by a butterfly
@@ -238,7 +393,8 @@ __device__ __forceinline__ void fa_decode_block(const AttnArgs &a, int split, in
         }
     }
     constexpr int NSL = NWV;
-    __shared__ float sm[NSL][R], sl[NSL][R], so[NSL][R][HD];
+    __shared__ float sm[NSL][R], sl[NSL][R];
+    __shared__ __attribute__((aligned(16))) float so[NSL][R][HD];
     if (kg == 0) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -247,149 +403,7 @@ __device__ __forceinline__ void fa_decode_block(const AttnArgs &a, int split, in
             for (int e = 0; e < 8; ++e) so[wave][r][dl * 8 + e] = o[r][e];
         }
     }
-    __syncthreads();
-    const int nrows = min(a.rows_per_group, rows_kv - r0);
-    for (int idx = tid; idx < R * HD; idx += NT) {
-        const int r = idx / HD, d = idx % HD;
-        if (r >= nrows) continue;
-        // max over the slots, then one weight per slot for its sum and output
-        // (independent terms, summed in slot order)
-        float mm = -INFINITY;
-        for (int sv = 0; sv < NSL; ++sv) mm = fmaxf(mm, sm[sv][r]);
-        const float mu = (mm == -INFINITY) ? 0.f : mm;
-        float ll = 0.f, oo = 0.f;
-        for (int sv = 0; sv < NSL; ++sv) {
-            const float wgt = fast_exp2(sm[sv][r] - mu);
-            ll = __builtin_fmaf(sl[sv][r], wgt, ll);
-            oo = __builtin_fmaf(so[sv][r][d], wgt, oo);
-        }
-        const int rr = r0 + r;
-        const int64_t head = hk * G + rr / LQ, qi = rr % LQ;
-        const int64_t grow = (b * a.hq + head) * a.l + qi;
-        if (a.splits == 1) {
-            const T ov = from_f32<T>(oo * (ll > 0.f ? 1.f / ll : 0.f));
-            const int64_t oidx = b * a.so0 + head * a.so1 + qi * a.so2 + d;
-            reinterpret_cast<T *>(a.O)[oidx] = ov;
-            if (a.lse && d == 0) a.lse[grow] = ll > 0.f ? (mm + __log2f(ll)) * kLn2 : -INFINITY;
-            continue;
-        }
-        if (!a.counters) {
-            // merged by the separate merge kernel
-            a.ws_o[(grow * a.splits + split) * HD + d] = oo;
-            if (d == 0) {
-                a.ws_ml[(grow * a.splits + split) * 2 + 0] = mm;
-                a.ws_ml[(grow * a.splits + split) * 2 + 1] = ll;
-            }
-            continue;
-        }
-        // agent-coherent stores (written through the XCD's L2): the
-        // work-group that merges the splits may run on another XCD
-        __hip_atomic_store(&a.ws_o[(grow * a.splits + split) * HD + d], oo, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        if (d == 0) {
-            __hip_atomic_store(&a.ws_ml[(grow * a.splits + split) * 2 + 0], mm, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&a.ws_ml[(grow * a.splits + split) * 2 + 1], ll, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    if (a.splits == 1 || !a.counters) return;
-
-    // The last of the group's split work-groups to arrive merges the splits
-    // in split order (bitwise repeatable whatever the arrival order).
-    // Ordering (as in the decode GEMM's merge): the split states are
-    // agent-scope relaxed atomic stores (`global_store sc1`, written through
-    // the per-XCD L2); each thread waits for their acknowledgements
-    // (s_waitcnt(0)) before the barrier that precedes tid 0's agent-scope
-    // counter RMW, and the merging work-group reads them with sc1 buffer
-    // loads, which miss the non-coherent caches.  This relies on the hardware
-    // rule that an acknowledged sc1 store is visible at the agent's coherence
-    // point before a later RMW of the same agent, not on a release / acquire
-    // pair (which would add an L2 write-back per XCD to every work-group).
-    __shared__ int s_last;
-    __shared__ float s_w[R][64];
-    __shared__ float s_M[R], s_L[R];
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    unsigned *ctr = a.counters + ((b * a.hkv + hk) * a.row_groups + rg) * kAttnCounterStride;
-    if (tid == 0)
-        s_last = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                 (unsigned)(a.splits - 1);
-    __syncthreads();
-    if (!s_last) return;
-    // The split states are read with agent-coherent (sc1) buffer loads, which
-    // unlike atomics can be batched.  Wave w turns row w's split maxima into
-    // weights (splits <= 64, one per lane); thread (r, d) then sums
-    // weight * o[split][d] in split order.
-    const __amdgpu_buffer_rsrc_t rs_ml = __builtin_amdgcn_make_buffer_rsrc((void *)a.ws_ml, (short)0, 0x7fffffff, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rs_o = __builtin_amdgcn_make_buffer_rsrc((void *)a.ws_o, (short)0, 0x7fffffff, 0x00020000);
-    constexpr int kSc1 = kSc1Aux;
-    auto grow_of = [&](int r) {
-        const int rr = r0 + r;
-        return (b * a.hq + hk * G + rr / LQ) * a.l + rr % LQ;
-    };
-    // Thread (r, d) = tid issues its o loads (at most 32 splits) before the
-    // weights are known, so both arrive in one memory round trip.
-    constexpr int kMaxSplits = 32;
-    float ov[kMaxSplits];
-    const bool pre = a.splits <= kMaxSplits && nrows * HD <= NT && tid < nrows * HD;
-    if (pre) {
-        const uint32_t base = (uint32_t)((grow_of(tid / HD) * a.splits * HD + tid % HD) * 4);
-#pragma unroll
-        for (int z = 0; z < kMaxSplits; ++z)
-            ov[z] = z < a.splits ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                       rs_o, base + (uint32_t)(z * HD * 4), 0, kSc1))
-                                 : 0.f;
-    }
-    for (int r = wave; r < nrows; r += NWV) {
-        const uint32_t base = (uint32_t)(grow_of(r) * a.splits * 2) * 4;
-        // (the b32 loads return raw bits)
-        const float mz = lane < a.splits
-                             ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_ml, base + lane * 8, 0, kSc1))
-                             : -INFINITY;
-        const float lz = lane < a.splits
-                             ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs_ml, base + lane * 8 + 4, 0, kSc1))
-                             : 0.f;
-        const float M = wave_max(mz);
-        const float Mu = (M == -INFINITY) ? 0.f : M;
-        const float w = lane < a.splits ? fast_exp2(mz - Mu) : 0.f;
-        s_w[r][lane] = w;
-        const float L = wave_sum(w * lz);
-        if (lane == 0) { s_M[r] = M; s_L[r] = L; }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < nrows * HD; idx += NT) {
-        const int r = idx / HD, d = idx % HD;
-        const int64_t grow = grow_of(r);
-        float acc = 0.f;
-        if (pre) {
-#pragma unroll
-            for (int z = 0; z < kMaxSplits; ++z)
-                if (z < a.splits) acc += s_w[r][z] * ov[z];
-        } else {
-            const uint32_t base = (uint32_t)((grow * a.splits * HD + d) * 4);
-            for (int z0 = 0; z0 < a.splits; z0 += 8) {
-                float o8[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    o8[j] = z0 + j < a.splits ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                                    rs_o, base + (uint32_t)((z0 + j) * HD * 4), 0, kSc1))
-                                              : 0.f;
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (z0 + j < a.splits) acc += s_w[r][z0 + j] * o8[j];
-            }
-        }
-        const float L = s_L[r];
-        const float inv = L > 0.f ? 1.f / L : 0.f;
-        const int rr = r0 + r;
-        const int64_t head = hk * G + rr / LQ, qi = rr % LQ;
-        T *Op = reinterpret_cast<T *>(a.O) + b * a.so0 + head * a.so1 + qi * a.so2;
-        Op[d] = from_f32<T>(acc * inv);
-        if (a.lse && d == 0) a.lse[grow] = L > 0.f ? (s_M[r] + __log2f(L)) * kLn2 : -INFINITY;
-    }
-    if (tid == 0) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    decode_finish<T, HD, R, NSL, NT>(a, split, b, hk, rg, r0, sm, sl, so);
 }
 
 // One query row (unit = KV head * row_groups + row, rows_per_group 1) over a

@@ -204,6 +204,38 @@ def test_sdpa_decode_vs_oracle(cuda, n, hq, hkv, l, s, d):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,hq,hkv,l,s,d", [
+    (2, 6, 2, 1, 1300, 64), (1, 40, 2, 1, 1025, 128),      # 3 rows; 20 rows: two row groups
+    (3, 8, 2, 4, 800, 128), (9, 32, 8, 1, 900, 128),       # 16 rows of 4 queries; 32 keys and one more per wave
+    (130, 16, 4, 1, 161, 64), (16, 8, 2, 1, 5000, 128)])   # one split; sixteen
+def test_sdpa_decode_mfma_rows(cuda, dtype, n, hq, hkv, l, s, d):
+    """Grouped-query decode on the MFMA kernel: device key counts from 0 to
+    the capacity with NaN in the cache past them, query rows that do not fill
+    a row group, strided caches.  |error| <= half an ulp of the result (2^-9
+    of |o| <= 5) plus the 2^-17 of the split probabilities: inside 1e-2."""
+    q = gen((n, hq, l, d), dtype, 61)
+    k, v = gen((n, s, hkv, d), dtype, 62).transpose(1, 2), gen((n, s, hkv, d), dtype, 63).transpose(1, 2)
+    g = torch.Generator().manual_seed(s)
+    lens = torch.randint(l, s + 1, (n,), generator=g).to(torch.int32)
+    lens[0] = s
+    if n > 2:
+        lens[1], lens[2] = (0 if l == 1 else l), l
+    kd, vd = k.to(cuda), v.to(cuda)
+    for b in range(n):
+        kd[b, :, lens[b]:] = float("nan")
+        vd[b, :, lens[b]:] = float("nan")
+    out, lse = ops.sdpa_decode(q.to(cuda), kd, vd, kv_len=lens.to(cuda), return_lse=True)
+    for b in sorted({0, 1 % n, 2 % n, n - 1}):
+        m = int(lens[b])
+        if m == 0:
+            assert not out[b].float().any() and bool(torch.isneginf(lse[b]).all())
+            continue
+        ref, lref = O.sdpa(npy(q[b:b + 1]), npy(k[b:b + 1, :, :m]), npy(v[b:b + 1, :, :m]), causal=True, align="bottom_right")
+        close(out[b:b + 1], ref)
+        np.testing.assert_allclose(npy(lse[b:b + 1]), lref, atol=1e-3, rtol=1e-4)
+
+
 def test_sdpa_decode_shapes_share_workspace(cuda):
     """Split calls of few and of many query rows in turn on one stream: no
     call's split states may land on another one's arrival counters."""
