@@ -165,8 +165,11 @@ def call(name: str, *args) -> None:
     check(name, getattr(load(), name)(*args))
 
 
+_I64x3 = ctypes.c_int64 * 3
+
+
 def strides3(*vals) -> ctypes.Array:
-    return (ctypes.c_int64 * 3)(*[int(v) for v in vals])
+    return _I64x3(*vals)
 
 
 def i64_array(vals) -> ctypes.Array:

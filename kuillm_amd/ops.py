@@ -13,6 +13,7 @@ stock PyTorch (the reference's dispatch contract, kuipy/__init__.py:53-75).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 
@@ -31,11 +32,25 @@ CHECK_INDEX = os.environ.get("KUIOPS_CHECK_INDEX", "0") == "1"
 
 
 def _lib_handle():
-    return _compile.load_library()
+    return _compile._loaded.get(_compile.LIB_NAME) or _compile.load_library()
+
+
+# The current stream's handle by device index, without the Stream object that
+# torch.cuda.current_stream builds (2 us of a ~10 us call; 0.1 us so).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    index = dev.index
+    if _raw_stream is None or index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(index)
+
+
+@functools.lru_cache(maxsize=4096)
+def _query_workspace(op: int, a: int, b: int, c: int) -> int:
+    """kuiops_query_workspace: a function of its arguments alone."""
+    return _lib_handle().kuiops_query_workspace(op, a, b, c)
 
 
 def _ptr(t) -> int | None:
@@ -75,7 +90,7 @@ def _stream_key(device: torch.device) -> int:
     """The stream a workspace is keyed on: torch's current stream on the device."""
     if device.type != "cuda":
         return 0
-    return torch.cuda.current_stream(device).cuda_stream
+    return _stream(device)
 
 
 def _capturing(device: torch.device) -> bool:
@@ -147,7 +162,7 @@ def _gemv(x, B, ldb, layout, bias, out):
     M, K = x.shape
     N = B.shape[1]
     lib = _lib_handle()
-    ws_bytes = lib.kuiops_query_workspace(_lib.OP_GEMV_SPLITK, M, N, K)
+    ws_bytes = _query_workspace(_lib.OP_GEMV_SPLITK, M, N, K)
     ws = workspace(x.device, ws_bytes, "gemv")
     _lib.check("kuiops_gemv_splitk", lib.kuiops_gemv_splitk(
         M, N, K, _dt(x.dtype), x.data_ptr(), x.stride(0), B.data_ptr(), ldb, layout,
@@ -176,7 +191,7 @@ def mm(A: torch.Tensor, B: torch.Tensor, out_dtype=None, gemv_max_m: int | None 
         except _lib.Unsupported:
             pass
     lib = _lib_handle()
-    ws_bytes = lib.kuiops_query_workspace(_lib.OP_ADDMM, M, N, K) if A.dtype in HALF else 0
+    ws_bytes = _query_workspace(_lib.OP_ADDMM, M, N, K) if A.dtype in HALF else 0
     if ws_bytes:
         # Too few output tiles to fill the GPU: the same kernels with split-K,
         # whose fp32 partials need a workspace (kuiops_mm takes none), through
@@ -209,7 +224,7 @@ def addmm(C: torch.Tensor, A: torch.Tensor, B: torch.Tensor, beta=1.0, alpha=1.0
     if beta == 0.0:
         c_kind, Cin, ldcin = _lib.C_NONE, None, 0
     elif C.dim() == 1 and C.shape[0] == N or (C.dim() == 2 and C.shape[0] == 1 and C.shape[1] == N):
-        c_kind, Cin, ldcin = _lib.C_ROW, C.reshape(N).contiguous(), 0
+        c_kind, Cin, ldcin = _lib.C_ROW, C if C.dim() == 1 and C.stride(0) == 1 else C.reshape(N).contiguous(), 0
     else:
         Cin = C.expand(M, N)
         if Cin.stride(1) != 1 or Cin.stride(0) < N:
@@ -226,7 +241,7 @@ def addmm(C: torch.Tensor, A: torch.Tensor, B: torch.Tensor, beta=1.0, alpha=1.0
         except _lib.Unsupported:
             pass
     lib = _lib_handle()
-    ws_bytes = lib.kuiops_query_workspace(_lib.OP_ADDMM, M, N, K)
+    ws_bytes = _query_workspace(_lib.OP_ADDMM, M, N, K)
     ws = workspace(A.device, ws_bytes) if ws_bytes else None
     _lib.check("kuiops_addmm", lib.kuiops_addmm(
         M, K, N, alpha, beta, _dt(A.dtype), A.data_ptr(), A.stride(0), B.data_ptr(), ldb, layout,
@@ -237,6 +252,8 @@ def addmm(C: torch.Tensor, A: torch.Tensor, B: torch.Tensor, beta=1.0, alpha=1.0
 
 def linear(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """x[..., K] @ W[N, K]^T (+ bias): nn.Linear with a K-contiguous weight."""
+    if x.dim() == 2:
+        return mm(x, W.t()) if bias is None else addmm(bias, x, W.t())
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
     if bias is None:
@@ -396,7 +413,7 @@ def sdpa(q, k, v, is_causal=False, scale=None, return_lse=True, decode_max_rows=
             b.data_ptr(), _lib.strides3(*b.stride()[:3]), _stream(q.device)))
         return out, lse
     if not is_causal and (hq // hkv) * l <= decode_max_rows and s > 0:
-        ws_bytes = lib.kuiops_query_workspace(_lib.OP_SDPA_DECODE, n * hq * l, s, ev)
+        ws_bytes = _query_workspace(_lib.OP_SDPA_DECODE, n * hq * l, s, ev)
         ws = workspace(q.device, ws_bytes, "attn")
         _lib.check("kuiops_sdpa_decode", lib.kuiops_sdpa_decode(
             n, hq, hkv, l, s, e, ev, _dt(q.dtype), q.data_ptr(), sq, k.data_ptr(), sk,
@@ -431,7 +448,7 @@ def sdpa_decode(q, k, v, scale=None, causal=True, return_lse=False, kv_len=None,
     if out.numel() == 0:
         return out, lse
     lib = _lib_handle()
-    ws_bytes = lib.kuiops_query_workspace(_lib.OP_SDPA_DECODE, n * hq * l, s, ev)
+    ws_bytes = _query_workspace(_lib.OP_SDPA_DECODE, n * hq * l, s, ev)
     ws = workspace(q.device, ws_bytes, "attn")
     _lib.check("kuiops_sdpa_decode", lib.kuiops_sdpa_decode(
         n, hq, hkv, l, s, e, ev, _dt(q.dtype), q.data_ptr(), _lib.strides3(*q.stride()[:3]),
@@ -649,7 +666,7 @@ def sort(x: torch.Tensor, dim: int = -1, descending: bool = False):
     inds = torch.empty(xc.shape, dtype=torch.int64, device=x.device)
     if vals.numel():
         lib = _lib_handle()
-        ws_bytes = lib.kuiops_query_workspace(_lib.OP_SORT, m, n, 0)
+        ws_bytes = _query_workspace(_lib.OP_SORT, m, n, 0)
         ws = workspace(x.device, ws_bytes) if ws_bytes else None
         _lib.check("kuiops_sort_lastdim", lib.kuiops_sort_lastdim(
             m, n, _dt(x.dtype), xc.data_ptr(), vals.data_ptr(), inds.data_ptr(), 1 if descending else 0,
@@ -742,7 +759,7 @@ def sample_top_p(scores: torch.Tensor, top_p: float, temperature: float = 1.0, g
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
     """2-D [m, n] view with unit column stride (copy otherwise)."""
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     return x2 if x2.stride(-1) == 1 else x2.contiguous()
 
 
@@ -755,8 +772,8 @@ def rmsnorm(x, weight, eps, residual=None, res_out=None, out=None):
     n = x.shape[-1]
     x2 = _rows(x)
     m = x2.shape[0]
-    r2 = None if residual is None else residual.reshape(-1, n)
-    ro2 = None if res_out is None else res_out.reshape(-1, n)
+    r2 = None if residual is None else residual if residual.dim() == 2 else residual.reshape(-1, n)
+    ro2 = None if res_out is None else res_out if res_out.dim() == 2 else res_out.reshape(-1, n)
     for t in (r2, ro2):
         if t is not None and (t.shape[0] != m or t.stride(-1) != 1 or t.dtype != x.dtype):
             raise _lib.KuiopsError("rmsnorm", _lib.E_INVALID)
@@ -1169,7 +1186,7 @@ def decode_rows_batched(x, W, x_kind="plain", out_kind="plain", in_add=None, nor
     elif out_kind == "swiglu":
         pair_off = N // 2
     lib = _lib_handle()
-    ws_bytes = lib.kuiops_query_workspace(_lib.OP_DECODE_ROWS_BATCHED, M, N, K) if split else 0
+    ws_bytes = _query_workspace(_lib.OP_DECODE_ROWS_BATCHED, M, N, K) if split else 0
     ws = workspace(x.device, ws_bytes, "decode_rows") if ws_bytes else None
     _lib.check("kuiops_decode_rows_batched", lib.kuiops_decode_rows_batched(
         M, N, K, _dt(x.dtype), _X_KIND[x_kind], _OUT_KIND[out_kind], x.data_ptr(), x.stride(0), _ptr(row), rows,
