@@ -147,9 +147,9 @@ KUIOPS_API int kuiops_bmm(int64_t batch, int64_t M, int64_t K, int64_t N, int in
 /* Skinny (decode) GEMM: out[M, N] = x[M, K] @ W[K, N] (+ bias[N]) for
  * 1 <= M <= 64, bf16/f16 in, fp32 accumulate, out_dtype = in or F32.
  * K is split over `splits` work-groups (0 = choose); fp32 partials go to the
- * workspace and are summed in split order (row-major W: by the last work-
- * group of each column strip to finish, K-contiguous W: by a second
- * kernel), so the result is bitwise repeatable.  Requires the workspace of
+ * workspace and are summed in split order (by the last work-group of each
+ * column strip to finish, or by a second kernel), so the result is bitwise
+ * repeatable.  Requires the workspace of
  * kuiops_query_workspace(KUIOPS_OP_GEMV_SPLITK, M, N, K).  Serves the
  * reference's mm/addmm families at decode shapes, which its gate rejects
  * (`M % 64`, kuipy/kuiops.py:372-374).                                    */

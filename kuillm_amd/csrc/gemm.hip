@@ -1385,7 +1385,7 @@ static bool dma_eligible(const GemmArgs &a, int64_t batch, bool bcol) {
 
 template <typename T, typename Tout>
 static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int splits_req, void *ws, size_t ws_bytes,
-                    hipStream_t st) {
+                    hipStream_t st, bool any_ws = false) {
     if constexpr (sizeof(Tout) == 2) {
         // short K (64 or 128), full 256x256 tiles, several tiles per CU: the
         // persistent kernel overlaps each tile's output stores with the next
@@ -1414,8 +1414,11 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
     int max_s = batch == 1 ? max_splits(a.M, a.N, a.K) : 1;
     const size_t part = (size_t)a.M * a.N * sizeof(float);
     if (splits_req == 0 && max_s > 1 && (!ws || ws_bytes < (size_t)max_s * part)) {
-        if (aligned) return KUIOPS_E_WORKSPACE;
-        max_s = 1;                  // (unaligned operands need no workspace)
+        if (aligned && !any_ws) return KUIOPS_E_WORKSPACE;
+        // (unaligned operands, and the decode GEMM, split as far as the
+        // workspace they were given allows)
+        max_s = ws && part > 0 ? (int)min((int64_t)max_s, (int64_t)(ws_bytes / part)) : 1;
+        if (max_s < 1) max_s = 1;
     }
     const TileChoice tc = choose_tile(a.M, a.N, a.K, batch, ws_ok ? max_s : 1,
                                       batch == 1 ? splits_req : 1);
@@ -1546,6 +1549,24 @@ static int gemm_entry(GemmArgs a, int64_t batch, int in_dt, int out_dt, int b_la
     if (in_dt == KUIOPS_F32 && out_dt == KUIOPS_F32) return run_f32(a, batch, bcol, st);
     if (in_dt == KUIOPS_F64 && out_dt == KUIOPS_F64) return run_simt<double, double, double>(a, batch, bcol, st);
     return KUIOPS_E_UNSUPPORTED;
+}
+
+// The decode GEMM's products on the tile kernel (aligned operands; the bias in
+// the output's type): see gemv.hip.
+int gemm_decode_tiles(int64_t M, int64_t N, int64_t K, int in_dt, const void *x, int64_t ldx, const void *W,
+                      int64_t ldw, bool wcol, const void *bias, int out_dt, void *out, int64_t ldo, void *ws,
+                      size_t ws_bytes, hipStream_t st) {
+    GemmArgs a{};
+    a.M = M; a.N = N; a.K = K;
+    a.A = x; a.lda = ldx; a.B = W; a.ldb = ldw;
+    a.out = out; a.ldo = ldo;
+    a.cin = bias; a.c_kind = bias ? KUIOPS_C_ROW : KUIOPS_C_NONE;
+    a.alpha = 1.f; a.beta = 1.f;
+    if (in_dt == KUIOPS_BF16)
+        return out_dt == KUIOPS_F32 ? run_mfma<bf16_t, float>(a, 1, wcol, true, 0, ws, ws_bytes, st, true)
+                                    : run_mfma<bf16_t, bf16_t>(a, 1, wcol, true, 0, ws, ws_bytes, st, true);
+    return out_dt == KUIOPS_F32 ? run_mfma<f16_t, float>(a, 1, wcol, true, 0, ws, ws_bytes, st, true)
+                                : run_mfma<f16_t, f16_t>(a, 1, wcol, true, 0, ws, ws_bytes, st, true);
 }
 
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {

@@ -702,6 +702,23 @@ static bool rows_eligible(const GemvArgs &a, bool wcol) {
     return true;
 }
 
+// Products that the MFMA tile kernel streams faster than the kernels here: every
+// K-contiguous W, whose 16 lanes x 16 bytes of a k step read 64-byte pieces of
+// 16 rows (gemv_splitk_kernel; us for M = 1 / 16 / 64, against the tile kernel:
+// 4096 x 4096 16.6 / 16.9 / 29.4 -> 11.0 / 11.5 / 13.2, 32000 x 2048 38 / 41 / 74
+// -> 32 / 32 / 33.5, 2048 x 5632 20.5 / 23.4 / 37 -> 9.9 / 10.3 / 11.9), and a
+// row-major W unless its strips or column blocks fill the CUs and x is short
+// (11008 x 4096, M = 1 / 16 / 64: 18.1 / 23.0 / 34.3 here, 22.2 / 21.5 / 26.3 there;
+// 2048 x 5632: 11.6 / 15.6 / 30.2 and 9.9 / 10.5 / 12.3).
+int gemm_decode_tiles(int64_t M, int64_t N, int64_t K, int in_dt, const void *x, int64_t ldx, const void *W,
+                      int64_t ldw, bool wcol, const void *bias, int out_dt, void *out, int64_t ldo, void *ws,
+                      size_t ws_bytes, hipStream_t st);
+
+static bool tiles_faster(int64_t M, int64_t N, int64_t K, bool wcol) {
+    if (wcol) return true;
+    return !((N >= 8192 && M <= 16) || (M == 1 && N >= 2048 && (N >= 4096 || K <= 4096)));
+}
+
 template <typename T, typename Tout>
 static int rows_dispatch(const GemvArgs &a, hipStream_t st) {
     dim3 grid((unsigned)cdiv(a.N, kRowsCB), (unsigned)a.splits);
@@ -804,46 +821,43 @@ static int gemv_run(int64_t M, int64_t N, int64_t K, int in_dtype, const void *x
     a.M = M; a.N = N; a.K = K;
     a.x = x; a.ldx = ldx; a.W = W; a.ldw = ldw; a.bias = bias;
     a.out = out; a.ldo = ldo;
-    hipStream_t st0 = as_stream(stream);
-    if (splits <= 0 && rows_eligible(a, wcol)) {
-        a.splits = rows_splits(N, K);
-        a.k_part = cdiv(cdiv(K, a.splits), 8) * 8;
-        a.splits = (int)cdiv(K, a.k_part);
-        if (a.splits > 1) {
-            const size_t need = kGemvCounterBytes + (size_t)a.splits * M * N * sizeof(float);
-            if (!workspace || workspace_bytes < need || !aligned16(workspace)) return KUIOPS_E_WORKSPACE;
-            a.counters = reinterpret_cast<unsigned *>(workspace);
-            a.partial = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + kGemvCounterBytes);
-            if (clear_counters) clear_counters_on(a.counters, cdiv(N, kRowsCB), st0);
-        }
-        if (in_dtype == KUIOPS_BF16)
-            return out_dtype == KUIOPS_F32 ? rows_dispatch<bf16_t, float>(a, st0) : rows_dispatch<bf16_t, bf16_t>(a, st0);
-        return out_dtype == KUIOPS_F32 ? rows_dispatch<f16_t, float>(a, st0) : rows_dispatch<f16_t, f16_t>(a, st0);
+    hipStream_t st = as_stream(stream);
+    const bool rows = splits <= 0 && rows_eligible(a, wcol), strip = !rows && splits <= 0 && strip_eligible(a, wcol);
+    int s = rows ? rows_splits(N, K) : strip ? strip_splits(N, K) : splits > 0 ? splits : gemv_choose_splits(M, N, K);
+    if (rows) {
+        a.k_part = cdiv(cdiv(K, s), 8) * 8;
+        s = (int)cdiv(K, a.k_part);
+    } else if (!strip) {
+        a.k_per_split = cdiv(cdiv(K, s), 128) * 128;
+        s = (int)cdiv(K, a.k_per_split);
     }
-    if (splits <= 0 && strip_eligible(a, wcol)) {
-        a.splits = strip_splits(N, K);
-        if (a.splits > 1) {
-            const size_t need = kGemvCounterBytes + (size_t)a.splits * M * N * sizeof(float);
-            if (!workspace || workspace_bytes < need || !aligned16(workspace)) return KUIOPS_E_WORKSPACE;
-            a.counters = reinterpret_cast<unsigned *>(workspace);
-            a.partial = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + kGemvCounterBytes);
-            if (clear_counters) clear_counters_on(a.counters, cdiv(N, kStripW), st0);
-        }
-        if (in_dtype == KUIOPS_BF16)
-            return out_dtype == KUIOPS_F32 ? strip_dispatch<bf16_t, float>(a, st0) : strip_dispatch<bf16_t, bf16_t>(a, st0);
-        return out_dtype == KUIOPS_F32 ? strip_dispatch<f16_t, float>(a, st0) : strip_dispatch<f16_t, f16_t>(a, st0);
-    }
-    int s = splits > 0 ? splits : gemv_choose_splits(M, N, K);
-    int64_t kps = cdiv(cdiv(K, s), 128) * 128;
-    s = (int)cdiv(K, kps);
     a.splits = s;
-    a.k_per_split = kps;
     if (s > 1) {
         const size_t need = kGemvCounterBytes + (size_t)s * M * N * sizeof(float);
         if (!workspace || workspace_bytes < need || !aligned16(workspace)) return KUIOPS_E_WORKSPACE;
+        a.counters = reinterpret_cast<unsigned *>(workspace);
         a.partial = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + kGemvCounterBytes);
     }
-    hipStream_t st = st0;
+    if (splits <= 0 && tiles_faster(M, N, K, wcol) && (!bias || out_dtype == in_dtype)) {
+        // (the partials behind the counters, within the size the query gives)
+        const size_t most = gemv_workspace_bytes(M, N, K);
+        const size_t have = workspace && aligned16(workspace) ? (workspace_bytes < most ? workspace_bytes : most) : 0;
+        const bool ws = have > kGemvCounterBytes;
+        return gemm_decode_tiles(M, N, K, in_dtype, x, ldx, W, ldw, wcol, bias, out_dtype, out, ldo,
+                                 ws ? reinterpret_cast<char *>(workspace) + kGemvCounterBytes : nullptr,
+                                 ws ? have - kGemvCounterBytes : 0, st);
+    }
+    if (s > 1 && clear_counters && (rows || strip)) clear_counters_on(a.counters, cdiv(N, rows ? kRowsCB : kStripW), st);
+    if (rows) {
+        if (in_dtype == KUIOPS_BF16)
+            return out_dtype == KUIOPS_F32 ? rows_dispatch<bf16_t, float>(a, st) : rows_dispatch<bf16_t, bf16_t>(a, st);
+        return out_dtype == KUIOPS_F32 ? rows_dispatch<f16_t, float>(a, st) : rows_dispatch<f16_t, f16_t>(a, st);
+    }
+    if (strip) {
+        if (in_dtype == KUIOPS_BF16)
+            return out_dtype == KUIOPS_F32 ? strip_dispatch<bf16_t, float>(a, st) : strip_dispatch<bf16_t, bf16_t>(a, st);
+        return out_dtype == KUIOPS_F32 ? strip_dispatch<f16_t, float>(a, st) : strip_dispatch<f16_t, f16_t>(a, st);
+    }
     if (in_dtype == KUIOPS_BF16)
         return out_dtype == KUIOPS_F32 ? gemv_dispatch<bf16_t, float>(a, wcol, st)
                                        : gemv_dispatch<bf16_t, bf16_t>(a, wcol, st);
