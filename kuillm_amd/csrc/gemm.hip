@@ -86,7 +86,7 @@ __device__ __forceinline__ u32x4 load8_any(const T *p, int64_t n) {
 
 // Operands of any stride and alignment, any K and N (an eager attention's
 // probabilities have rows as long as the prompt), 64-bit addresses.  It took
-// over from a SIMT kernel: bmm 32 x 777x777x128 bf16 183 -> 27 us.  What
+// over from a SIMT kernel: bmm 32 x 777x777x128 bf16 183 -> 24 us.  What
 // bounds it: each stage waits for its loads, one stage ahead in registers.
 template <typename T, int BM, int BN, int WM, int WN, bool BCOL, typename Tout, bool SPLIT>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
@@ -1351,9 +1351,16 @@ static void launch_reduce(const GemmArgs &a, hipStream_t st) {
     else hipLaunchKernelGGL((splitk_reduce_kernel<Tout, false>), grid, dim3(256), 0, st, a);
 }
 
+// 64x128 tiles where 128x128 ones would leave a CU fewer than two (32 x
+// 777x777x128 27 -> 24 us, 8 x 333x333x128 16.3 -> 11.2).
 template <typename T, typename Tout, bool SPLIT>
-static void launch_mfma(const GemmArgs &a, bool bcol, int64_t gz, hipStream_t st) {
+static void launch_mfma(int bm, const GemmArgs &a, bool bcol, int64_t gz, hipStream_t st) {
     dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n), (unsigned)gz);
+    if (bm == 64) {
+        if (bcol) hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 128, 2, 2, true, Tout, SPLIT>), grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 128, 2, 2, false, Tout, SPLIT>), grid, dim3(256), 0, st, a);
+        return;
+    }
     if (bcol) hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 2, 2, true, Tout, SPLIT>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 2, 2, false, Tout, SPLIT>), grid, dim3(256), 0, st, a);
 }
@@ -1458,7 +1465,8 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
         return launch_status();
     }
     const bool tile_ok = aligned && a.K > 0 && offsets_fit(a, bcol);
-    const int bk = tile_ok ? kTiles[tc.tile].bk : 64, bm = tile_ok ? kTiles[tc.tile].bm : 128,
+    const int64_t t128 = cdiv(a.M, 128) * cdiv(a.N, 128) * batch;
+    const int bk = tile_ok ? kTiles[tc.tile].bk : 64, bm = tile_ok ? kTiles[tc.tile].bm : t128 < 2 * num_cus() ? 64 : 128,
               bn = tile_ok ? kTiles[tc.tile].bn : 128;
     int splits = tile_ok ? tc.splits : (splits_req > 0 ? splits_req : max_s);
     if (batch != 1) splits = 1;
@@ -1482,9 +1490,9 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
         if (splits > 1) launch_tile<T, Tout, true>(tc.tile, a, bcol, grid, st);
         else launch_tile<T, Tout, false>(tc.tile, a, bcol, grid, st);
     } else if (splits > 1) {
-        launch_mfma<T, Tout, true>(a, bcol, splits, st);
+        launch_mfma<T, Tout, true>(bm, a, bcol, splits, st);
     } else {
-        launch_mfma<T, Tout, false>(a, bcol, batch, st);
+        launch_mfma<T, Tout, false>(bm, a, bcol, batch, st);
     }
     if (splits > 1) launch_reduce<Tout>(a, st);
     return launch_status();

@@ -164,7 +164,8 @@ def test_addmm_tile_kernel_edges(cuda, layout, M, N, K):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,M,K,N", [(5, 77, 77, 64), (3, 130, 201, 131), (2, 1, 7, 9), (4, 333, 129, 128), (1, 257, 1031, 255)])
+@pytest.mark.parametrize("b,M,K,N", [(5, 77, 77, 64), (3, 130, 201, 131), (2, 1, 7, 9), (4, 333, 129, 128), (1, 257, 1031, 255),
+                                     (45, 500, 67, 260)])      # 128x128 tiles; the others 64x128
 @pytest.mark.parametrize("layout", ["row", "col"])
 def test_bmm_odd_strides(cuda, dtype, b, M, K, N, layout):
     """Rows of odd length at 2-byte alignment: slices of wider NaN-filled
