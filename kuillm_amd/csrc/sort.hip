@@ -10,7 +10,7 @@
 //   final rank = its position in its own chunk + the number of smaller keys in
 //   every other chunk (a binary search of each other chunk, staged in LDS in
 //   turn) and writes value and index there.  For rows of up to 32 chunks the
-//   searches run one work-group per (chunk, other chunk) pair and a third
+//   searches run one work-group per (chunk, group of other chunks) and a third
 //   pass sums each key's counts and scatters.  Values are copied bit-exactly.
 // cumsum: one 1024-thread work-group per row, tiles of 4096 elements (four
 //   consecutive per thread, coalesced), block scans plus a running carry
@@ -210,49 +210,64 @@ __global__ __launch_bounds__(kSortThreads) void sort_rank_kernel(int64_t n, int 
     }
 }
 
-// Pass 2, wide form (rows of at most kSortWideChunks chunks): one
-// work-group per (own chunk c, other chunk o) counts, for every key of
-// chunk c, the keys of chunk o below it (a binary search of chunk o staged
-// in LDS; o == c: the key's own position), into part[row][o][c][p].  All
-// nc^2 searches run at once instead of nc - 1 in turn per work-group.
-constexpr int kSortWideChunks = 32;
+// Pass 2, wide form (rows of at most kSortWideChunks chunks): work-group (own
+// chunk c, group g of `per` other chunks) counts, for every key of chunk c,
+// the keys of those chunks below it (a binary search of each in LDS, the next
+// one loading meanwhile; c itself: the key's own position), into
+// part[row][g][c][p].  One chunk per group while the pairs alone fill the GPU's
+// work-groups (a single row: all nc^2 searches at once); more with more rows,
+// so that the counts written here and read by pass 3 stay small (8 rows of
+// 32000: 33 MB with one chunk per group, rank + scatter 25 + 20 us; about
+// 20 together with 8).  What bounds it: the searches' LDS reads, two keys' at a time.
+constexpr int kSortWideChunks = 32, kSortMaxPer = 8;
 template <int CH>
-__global__ __launch_bounds__(CH / 2) void sort_rank_part_kernel(int nchunks, const uint64_t *ws, uint32_t *part) {
+__global__ __launch_bounds__(CH / 2) void sort_rank_part_kernel(int nchunks, int per, const uint64_t *ws, uint32_t *part) {
     constexpr int NT = CH / 2;
-    __shared__ uint64_t s[CH];
-    const int tid = threadIdx.x, c = blockIdx.x, o = blockIdx.y;
+    __shared__ uint64_t s[2][CH];
+    const int tid = threadIdx.x, c = blockIdx.x, g = blockIdx.y;
     const int64_t row = blockIdx.z;
     const uint64_t *base = ws + row * nchunks * (int64_t)CH;
-    uint32_t *out = part + ((row * nchunks + o) * nchunks + c) * (int64_t)CH;
-    if (o == c) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) out[tid + h * NT] = tid + h * NT;
-        return;
-    }
-    uint64_t mine[2];
+    uint32_t *out = part + ((row * gridDim.y + g) * nchunks + c) * (int64_t)CH;
+    const int o0 = g * per, o1 = min(nchunks, o0 + per);
+    uint64_t mine[2], nxt[2];
+    uint32_t rank[2] = {0, 0};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        s[tid + h * NT] = base[(int64_t)o * CH + tid + h * NT];
         mine[h] = base[(int64_t)c * CH + tid + h * NT];
+        nxt[h] = base[(int64_t)o0 * CH + tid + h * NT];
     }
-    __syncthreads();
+    for (int o = o0; o < o1; ++o) {
+        uint64_t *t = s[(o - o0) & 1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        // keys are unique; padding ~0 is above every real key
-        int lo = 0, hi = CH;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (s[mid] < mine[h]) lo = mid + 1;
-            else hi = mid;
+        for (int h = 0; h < 2; ++h) t[tid + h * NT] = nxt[h];
+        __syncthreads();            // (the other buffer's readers are past it by now)
+        if (o + 1 < o1) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) nxt[h] = base[(int64_t)(o + 1) * CH + tid + h * NT];
         }
-        out[tid + h * NT] = (uint32_t)lo;
+        if (o == c) {
+            rank[0] += tid;
+            rank[1] += tid + NT;
+            continue;
+        }
+        // keys are unique; padding ~0 is above every real key
+        int p0 = 0, p1 = 0;
+#pragma unroll
+        for (int step = CH / 2; step > 0; step >>= 1) {
+            if (t[p0 + step - 1] < mine[0]) p0 += step;
+            if (t[p1 + step - 1] < mine[1]) p1 += step;
+        }
+        rank[0] += p0 + (t[p0] < mine[0] ? 1 : 0);
+        rank[1] += p1 + (t[p1] < mine[1] ? 1 : 0);
     }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) out[tid + h * NT] = rank[h];
 }
 
-// Pass 3, wide form: each key's rank is the sum of its nc partial counts;
+// Pass 3, wide form: each key's rank is the sum of its `ng` partial counts;
 // value and index go there.
 template <typename T, int CH>
-__global__ __launch_bounds__(CH / 2) void sort_scatter_kernel(int64_t n, int nchunks, const T *X, T *vals,
+__global__ __launch_bounds__(CH / 2) void sort_scatter_kernel(int64_t n, int nchunks, int ng, const T *X, T *vals,
                                                                int64_t *inds, const uint64_t *ws,
                                                                const uint32_t *part) {
     constexpr int NT = CH / 2;
@@ -265,12 +280,12 @@ __global__ __launch_bounds__(CH / 2) void sort_scatter_kernel(int64_t n, int nch
         const int p = tid + h * NT;
         const uint64_t key = keys[p];
         if (key == ~0ull) continue;                  // padding
-        // (all nc counts load at once: the loop is unrolled to the chunk limit)
+        // (all counts load at once: the loop is unrolled to the chunk limit)
         uint32_t rank = 0;
-        const uint32_t *pp = part + (row * nchunks * nchunks + c) * (int64_t)CH + p;
+        const uint32_t *pp = part + (row * ng * nchunks + c) * (int64_t)CH + p;
 #pragma unroll
         for (int o = 0; o < kSortWideChunks; ++o)
-            if (o < nchunks) rank += pp[(int64_t)o * nchunks * CH];
+            if (o < ng) rank += pp[(int64_t)o * nchunks * CH];
         const int64_t src = (int64_t)(uint32_t)key;
         vals[row * n + rank] = x[src];
         inds[row * n + rank] = src;
@@ -696,16 +711,20 @@ extern "C" int kuiops_sort_lastdim(int64_t m, int64_t n, int dtype, const void *
     uint32_t *part = wide ? reinterpret_cast<uint32_t *>(ws + (size_t)m * nc * ch) : nullptr;
     hipStream_t st = as_stream(stream);
     const dim3 grid((unsigned)nc, (unsigned)m);
-    const dim3 pairs((unsigned)nc, (unsigned)nc, (unsigned)m);
+    // other chunks per rank work-group: about 1024 work-groups
+    const int64_t pairs_all = m * nc64 * nc64;
+    const int per = (int)(pairs_all <= 1024 ? 1 : pairs_all / 1024 < kSortMaxPer ? pairs_all / 1024 : kSortMaxPer);
+    const int ng = (nc + per - 1) / per;
+    const dim3 pairs((unsigned)nc, (unsigned)ng, (unsigned)m);
 #define KUIOPS_SORT_CH(T, CH)                                                                                 \
     do {                                                                                                      \
         hipLaunchKernelGGL((sort_chunk_kernel<T, CH>), grid, dim3(CH / 2), 0, st, n, nc, (const T *)X,       \
                            (T *)values, indices, ws, descending);                                              \
         if (wide) {                                                                                           \
-            hipLaunchKernelGGL((sort_rank_part_kernel<CH>), pairs, dim3(CH / 2), 0, st, nc,                   \
+            hipLaunchKernelGGL((sort_rank_part_kernel<CH>), pairs, dim3(CH / 2), 0, st, nc, per,              \
                                (const uint64_t *)ws, part);                                                   \
-            hipLaunchKernelGGL((sort_scatter_kernel<T, CH>), grid, dim3(CH / 2), 0, st, n, nc, (const T *)X,  \
-                               (T *)values, indices, (const uint64_t *)ws, (const uint32_t *)part);          \
+            hipLaunchKernelGGL((sort_scatter_kernel<T, CH>), grid, dim3(CH / 2), 0, st, n, nc, ng,            \
+                               (const T *)X, (T *)values, indices, (const uint64_t *)ws, (const uint32_t *)part);          \
         } else if (nc > 1) {                                                                                  \
             hipLaunchKernelGGL(sort_rank_kernel<T>, grid, dim3(kSortThreads), 0, st, n, nc, (const T *)X,     \
                                (T *)values, indices, (const uint64_t *)ws);                                   \

@@ -208,7 +208,8 @@ def test_sort_golden(cuda, golden):
                                        (5, 1, torch.float32), (4, 7000, torch.bfloat16), (2, 513, torch.float16),
                                        (1, 131072, torch.float32),
                                        (17, 65536, torch.bfloat16),    # 32 chunks x 17 rows: the per-chunk rank pass
-                                       (20, 32000, torch.float32)])    # 2048-key chunks, pairwise rank pass
+                                       (9, 20000, torch.float32), (64, 8193, torch.float32),    # 3 and 5 chunks per rank group, the last one short
+                                       (20, 32000, torch.float32)])    # 2048-key chunks, 5 of them per rank group
 def test_sort_vs_oracle(cuda, m, n, dtype):
     g = torch.Generator().manual_seed(n)
     x = (torch.randn(m, n, generator=g) * 4).to(dtype)
