@@ -25,6 +25,8 @@
 //   KV head (grouped-query attention), keeps fp32 online-softmax state per
 //   row and writes (max, sum, unnormalised output) to the workspace; the last
 //   work-group of a row group to finish merges the splits in split order.
+//   With 3 or more query rows per KV head: fa_decode_mfma_kernel, 16 rows per
+//   work-group on MFMAs, the same split states and merge.
 //
 // Semantics: aten scaled_dot_product_attention (the reference's fallthrough,
 // kuipy/kuiops.py:627-681 rejects is_causal; tests/test_jit_ops.py:173-193).

@@ -9,10 +9,13 @@
 //     64-column strip, streams its rows through LDS by buffer DMA and feeds
 //     16x16x32 MFMAs with x as the A operand (transposing LDS reads give the
 //     W operand); the waves' K ranges are summed in LDS in wave order.
-//   * gemv_splitk_kernel (K-contiguous W, i.e. an nn.Linear weight seen
-//     through .t(), or shapes the others refuse): one 16-byte load per lane is
-//     already an MFMA operand; `splits` work-groups share a strip and
-//     gemv_reduce_kernel sums their partials in split order.
+//   * gemm_tile_kernel (gemm_tile.hpp; K-contiguous W, i.e. an nn.Linear weight
+//     seen through .t(), and a row-major W too narrow for the kernels above to
+//     fill the CUs: tiles_faster).
+//   * gemv_splitk_kernel (a caller's own split count, fp32 outputs with a bias):
+//     one 16-byte load per lane is already an MFMA operand; `splits`
+//     work-groups share a strip and gemv_reduce_kernel sums their partials in
+//     split order.
 //
 // Wherever K is split over work-groups the partials are summed in split
 // order 0..splits-1, so results are bitwise repeatable.
