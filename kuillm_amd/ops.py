@@ -772,8 +772,7 @@ def rmsnorm(x, weight, eps, residual=None, res_out=None, out=None):
     n = x.shape[-1]
     x2 = _rows(x)
     m = x2.shape[0]
-    r2 = None if residual is None else residual if residual.dim() == 2 else residual.reshape(-1, n)
-    ro2 = None if res_out is None else res_out if res_out.dim() == 2 else res_out.reshape(-1, n)
+    r2, ro2 = (t if t is None or t.dim() == 2 and t.shape[1] == n else t.reshape(-1, n) for t in (residual, res_out))
     for t in (r2, ro2):
         if t is not None and (t.shape[0] != m or t.stride(-1) != 1 or t.dtype != x.dtype):
             raise _lib.KuiopsError("rmsnorm", _lib.E_INVALID)

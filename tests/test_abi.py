@@ -174,3 +174,52 @@ def test_decode_step_host_checks(lib):
     assert sup(L, d, ffn, 16, hkv, 128, 32000, 385, _lib.BF16) == _lib.E_UNSUPPORTED
     assert sup(L, d, ffn, hq, hkv, hd, 32000, 640, _lib.F32) == _lib.E_UNSUPPORTED
     assert sup(L, d, ffn, hq, hkv, hd, 32000, 0, _lib.BF16) == _lib.E_INVALID
+
+
+class _RmsNormCalls:
+    """Stands in for the library: records kuiops_rmsnorm's arguments, launches nothing."""
+
+    def __init__(self):
+        self.calls = []
+
+    def kuiops_rmsnorm(self, *args):
+        self.calls.append(args)
+        return _lib.OK
+
+
+@pytest.mark.parametrize("shape, ok", [
+    ((4, 64), True), ((2, 2, 64), True), ((8, 32), True), ((4, 1, 64), True),
+    ((4, 32), False), ((4, 128), False), ((2, 128, 2), False), ((8, 64), False), ((4, 64, 2), False),
+])
+@pytest.mark.parametrize("which", ["residual", "res_out"])
+def test_rmsnorm_refuses_other_row_widths(monkeypatch, shape, ok, which):
+    """x [4, 64]: a residual / res_out is taken when its elements form 4 rows
+    of 64; one of another width would be read or written past its rows."""
+    import torch
+
+    from kuillm_amd import ops
+    stub = _RmsNormCalls()
+    monkeypatch.setattr(ops, "_lib_handle", lambda: stub)
+    monkeypatch.setattr(ops, "_stream", lambda dev: 0)
+    bf = torch.bfloat16
+    x, w, t = torch.zeros(4, 64, dtype=bf), torch.ones(64, dtype=bf), torch.zeros(shape, dtype=bf)
+    if not ok:
+        with pytest.raises(_lib.KuiopsError):
+            ops.rmsnorm(x, w, 1e-5, **{which: t})
+        assert not stub.calls
+        return
+    ops.rmsnorm(x, w, 1e-5, **{which: t})
+    ptr, ld = stub.calls[0][5:7] if which == "residual" else stub.calls[0][7:9]
+    assert (ptr, ld) == (t.data_ptr(), 64)
+
+
+def test_rmsnorm_refuses_overlapping_rows(lib):
+    p = ctypes.c_void_p(1 << 20)
+
+    def call(m, ldr, ldro):
+        return lib.kuiops_rmsnorm(m, 64, _lib.BF16, p, 64, p if ldr is not None else None, ldr or 0,
+                                  p if ldro is not None else None, ldro or 0, p, 1e-5, p, 64, None)
+
+    for ldr, ldro in ((32, None), (-64, None), (None, 32), (None, 0), (64, 32)):
+        assert call(4, ldr, ldro) == _lib.E_INVALID
+        assert call(0, ldr, ldro) == _lib.OK
