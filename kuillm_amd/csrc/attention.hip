@@ -469,13 +469,67 @@ __global__ __launch_bounds__(128) void fa_decode_combine_kernel(AttnArgs a) {
 //     it in every lane of a key's group).
 //   * O^T += V^T P^T: V goes to LDS by DMA and is read transposed
 //     (ds_read_b64_tr_b16; keys numbered in the order the score accumulator
-//     holds them).  P stays exact to fp32 rounding of the result: it is the
-//     sum of two 16-bit halves (P = hi + lo, 2^-17 relative for bf16), one MFMA each.
+//     holds them).  P is the sum of three 16-bit parts, one MFMA each, so no
+//     bit of the fp32 probability is lost: see ProbSplit.
 // K and V descriptors end at the sequence's key count (device memory), so keys
 // past it are neither fetched nor seen, and its keys are spread evenly over
 // the splits.  What bounds it: the K / V stream (16 sequences of 2000-4000
 // keys, GQA 32/8, head dim 128: 57 us for the VALU form, which also read the
-// caches to their capacity, 44.5 now).
+// caches to their capacity, 43.7 now).
+//
+// ProbSplit: a probability p as three values of T, each the leading bits of
+// what is left, cut off and not rounded, so that none is negative and an
+// infinite V gives an infinite sum, not inf - inf.  p is relative to m_used +
+// kShift, so p <= 2^(kRescaleSlack - kShift).
+//   bf16: 8 + 8 + 8 bits, p exactly.  Zero parts of a p > 0 are raised to
+//     2^-126 (0 x inf is NaN).  p <= 1.
+//   f16: 11 + 11 + 2 bits down to f16's smallest step 2^-24; p <= 2^15 puts
+//     that at 2^-31 of the row's largest.  A zero part raised to it would
+//     count (16384 unlikely keys: 2^-16), so that is done only in a second
+//     pass over the wave's keys, made when the first one's sums are not finite.
+// Against two rounded halves (2^-17 for bf16, and for f16 2^-25 of the largest)
+// it takes 0-4% longer in bf16, up to 7% in f16 (us: 16 sequences of 4000 keys
+// 43.5 / 43.7 / 44.2, 8 of 1024 11.5 / 11.8 / 12.3, head dim 64, 64 of 640 15.5 /
+// 16.0 / 16.2).
+template <typename T> struct ProbSplit;
+template <> struct ProbSplit<bf16_t> {
+    typedef bf16_t t2 __attribute__((ext_vector_type(2)));
+    static constexpr float kShift = kRescaleSlack;
+    static constexpr bool kTwoPass = false;
+    static __device__ __forceinline__ float cut(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+    static __device__ __forceinline__ void split(float p0, float p1, bool, t2 &hi, t2 &mid, t2 &lo) {
+        const float p[2] = {p0, p1};
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float h = cut(p[e]), r = p[e] - h, m = cut(r), f = fminf(p[e], 0x1p-126f);
+            hi[e] = (bf16_t)h;
+            mid[e] = (bf16_t)fmaxf(m, f);
+            lo[e] = (bf16_t)fmaxf(r - m, f);
+        }
+    }
+};
+template <> struct ProbSplit<f16_t> {
+    typedef f16_t t2 __attribute__((ext_vector_type(2)));
+    static constexpr float kShift = kRescaleSlack - 15.f;
+    static constexpr bool kTwoPass = true;
+    static __device__ __forceinline__ void split(float p0, float p1, bool raise, t2 &hi, t2 &mid, t2 &lo) {
+        hi = __builtin_bit_cast(t2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+        const float r0 = p0 - (float)hi[0], r1 = p1 - (float)hi[1];
+        mid = __builtin_bit_cast(t2, __builtin_amdgcn_cvt_pkrtz(r0, r1));
+        lo = t2{(f16_t)(r0 - (float)mid[0]), (f16_t)(r1 - (float)mid[1])};
+        if (raise) {
+            const float p[2] = {p0, p1};
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const f16_t f = p[e] > 0.f ? (f16_t)0x1p-24f : (f16_t)0.f;
+                hi[e] = hi[e] < f ? f : hi[e];      // (a NaN stays)
+                mid[e] = mid[e] < f ? f : mid[e];
+                lo[e] = lo[e] < f ? f : lo[e];
+            }
+        }
+    }
+};
+
 template <typename T, int HD>
 __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(AttnArgs a) {
     constexpr int NWV = 4, KB = 32, R = 16;
@@ -559,6 +613,8 @@ __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(AttnArgs a) {
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_used = -INFINITY, l_run = 0.f;
+    typedef ProbSplit<T> Split;
+    bool raise = false;
     auto step = [&](int k0, int slot, const char *sv) __attribute__((always_inline)) {
         f32x4 sc[2];
 #pragma unroll
@@ -587,19 +643,26 @@ __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(AttnArgs a) {
                 for (int i = 0; i < 4; ++i) o[t][i] *= alpha;
             m_used = m_new;
         }
-        const float mref = m_used == -INFINITY ? 0.f : m_used;
+        const float mref = m_used == -INFINITY ? 0.f : m_used + Split::kShift;
         typedef T t8 __attribute__((ext_vector_type(8)));
-        t8 hi, lo;
+        t8 hi, mid, lo;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float p = fast_exp2(sc[t][i] - mref);
-                l_run += p;
-                hi[4 * t + i] = from_f32<T>(p);
-                lo[4 * t + i] = from_f32<T>(p - to_f32(hi[4 * t + i]));
+            for (int i = 0; i < 4; i += 2) {
+                const float p0 = fast_exp2(sc[t][i] - mref), p1 = fast_exp2(sc[t][i + 1] - mref);
+                l_run += p0;
+                l_run += p1;
+                typename Split::t2 h2, m2, l2;
+                Split::split(p0, p1, raise, h2, m2, l2);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    hi[4 * t + i + e] = h2[e];
+                    mid[4 * t + i + e] = m2[e];
+                    lo[4 * t + i + e] = l2[e];
+                }
             }
-        const frag fh = __builtin_bit_cast(frag, hi), fl = __builtin_bit_cast(frag, lo);
+        const frag fh = __builtin_bit_cast(frag, hi), fm = __builtin_bit_cast(frag, mid), fl = __builtin_bit_cast(frag, lo);
         // this step's V tile has landed: only the next step's loads are younger
         constexpr int Y = 2 * KK + DV;
         __builtin_amdgcn_s_waitcnt((Y & 15) | ((Y >> 4) << 14) | (7 << 4) | (15 << 8));
@@ -614,32 +677,52 @@ __global__ __launch_bounds__(256) void fa_decode_mfma_kernel(AttnArgs a) {
             const u32x2 h0 = __builtin_bit_cast(u32x2, t0), h1 = __builtin_bit_cast(u32x2, t1);
             const frag vf = as_frag<frag>(u32x4{h0[0], h0[1], h1[0], h1[1]});
             o[dt] = Mfma<T>::m16(vf, fh, o[dt]);
+            o[dt] = Mfma<T>::m16(vf, fm, o[dt]);
             o[dt] = Mfma<T>::m16(vf, fl, o[dt]);
         }
     };
 
     constexpr int KS = NWV * KB;
-    int k0 = kbeg + wave * KB;
-    issue(k0, 0, sV0);
-    for (; k0 < kend; k0 += 2 * KS) {
-        issue(k0 + KS, 1, sV1);
-        step(k0, 0, sV0);
-        // (this wave's reads of the tile are done before its refill)
-        __builtin_amdgcn_s_waitcnt(0xc07f);
+    for (;;) {
+        int k0 = kbeg + wave * KB;
+        issue(k0, 0, sV0);
+        for (; k0 < kend; k0 += 2 * KS) {
+            issue(k0 + KS, 1, sV1);
+            step(k0, 0, sV0);
+            // (this wave's reads of the tile are done before its refill)
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            __builtin_amdgcn_sched_barrier(0);
+            issue(k0 + 2 * KS, 0, sV0);
+            step(k0 + KS, 1, sV1);
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // no DMA is in flight past here: the wave's state takes the place of
+        // its first V tile, a second pass fills it again
+        __builtin_amdgcn_s_waitcnt(0);
         __builtin_amdgcn_sched_barrier(0);
-        issue(k0 + 2 * KS, 0, sV0);
-        step(k0 + KS, 1, sV1);
-        __builtin_amdgcn_s_waitcnt(0xc07f);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (Split::kTwoPass) {
+            float z = 0.f;              // stays 0 if every sum is finite
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) z = __builtin_fmaf(o[t][i], 0.f, z);
+            if (!raise && __any(row_ok && z != 0.f)) {
+                raise = true;
+                m_used = -INFINITY;
+                l_run = 0.f;
+#pragma unroll
+                for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                continue;
+            }
+        }
+        break;
     }
-    // the wave's state takes the place of its first V tile, once its DMA is done
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_sched_barrier(0);
     float (*so)[R][HD] = reinterpret_cast<float (*)[R][HD]>(sV0);
     // lanes of a row hold disjoint keys: row sums over the lane groups
     l_run = xor_add<32>(xor_add<16>(l_run));
     if (G4 == 0) {
-        sm[wave][lr] = m_used;
+        sm[wave][lr] = m_used + Split::kShift;
         sl[wave][lr] = l_run;
     }
 #pragma unroll

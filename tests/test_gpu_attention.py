@@ -213,7 +213,7 @@ def test_sdpa_decode_mfma_rows(cuda, dtype, n, hq, hkv, l, s, d):
     """Grouped-query decode on the MFMA kernel: device key counts from 0 to
     the capacity with NaN in the cache past them, query rows that do not fill
     a row group, strided caches.  |error| <= half an ulp of the result (2^-9
-    of |o| <= 5) plus the 2^-17 of the split probabilities: inside 1e-2."""
+    of |o| <= 5): inside 1e-2."""
     q = gen((n, hq, l, d), dtype, 61)
     k, v = gen((n, s, hkv, d), dtype, 62).transpose(1, 2), gen((n, s, hkv, d), dtype, 63).transpose(1, 2)
     g = torch.Generator().manual_seed(s)
@@ -234,6 +234,72 @@ def test_sdpa_decode_mfma_rows(cuda, dtype, n, hq, hkv, l, s, d):
         ref, lref = O.sdpa(npy(q[b:b + 1]), npy(k[b:b + 1, :, :m]), npy(v[b:b + 1, :, :m]), causal=True, align="bottom_right")
         close(out[b:b + 1], ref)
         np.testing.assert_allclose(npy(lse[b:b + 1]), lref, atol=1e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_sdpa_decode_probability_bits(cuda, dtype):
+    """The probabilities that multiply V hold the bits of an fp32 number.  In
+    each sequence A keys have score 0 and V = 1, B keys score a and V = -v,
+    with A, B and v such that the result nearly cancels: an error of the
+    probability exp(a), the same for its B keys, is not hidden by the rounding
+    of the result.  Relative errors of exp(a): the score times log2 e (|a|
+    2^-23), exp2 (2^-23), and for f16 a step of 2^-31 of the largest
+    probability, half of it per key; the sums add 2^-22."""
+    rng = np.random.default_rng(7)
+    s, d = 2048, 64
+    scores = [-0.23, -0.61, -0.97, -1.33, -1.8, -2.6] if dtype == torch.bfloat16 else [-0.61, -1.8, -6.3, -7.1, -7.7, -8.4]
+    eps, n = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10, len(scores)
+    k, v, bounds = torch.zeros(n, 1, s, d), torch.zeros(n, 1, s, d), []
+    grid = np.concatenate([2.0 ** e * (1 + eps * np.arange(int(1 / eps))) for e in range(-2, 4)])
+    for b, a in enumerate(scores):
+        a = float(torch.tensor(a).to(dtype))
+        best = min(((abs(A - (s - A) * math.exp(a) * w) / (A + (s - A) * math.exp(a)), A, w)
+                    for A in range(1, s // 2, 7) for w in (grid[np.abs(A - (s - A) * math.exp(a) * grid).argmin()],)))
+        _, A, w = best
+        at = rng.permutation(s)
+        k[b, 0, at[A:], 0] = a
+        v[b, 0] = 1.0
+        v[b, 0, at[A:]] = -float(w)
+        share = (s - A) / (A + (s - A) * math.exp(a))
+        err = math.exp(a) * (abs(a) * 2.0 ** -23 + 2.0 ** -23) + (2.0 ** -32 if dtype == torch.float16 else 0)
+        bounds.append(share * err * (1 + w) + 2.0 ** -22)
+    q = torch.zeros(n, 4, 1, d)
+    q[..., 0] = 1.0
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    out = ops.sdpa_decode(q.to(cuda), k.to(cuda), v.to(cuda), scale=1.0)[0].double().cpu()
+    p = torch.softmax(k[:, 0, :, 0].double(), -1)
+    ref = (p[:, None] @ v[:, 0].double()).view(n, 1, 1, d)
+    assert ref.abs().max() < 5e-4
+    err = (out - ref).abs().amax((1, 2, 3))
+    assert (err <= torch.tensor(bounds) + eps * ref.abs().amax((1, 2, 3))).all(), (err, bounds)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_sdpa_decode_infinite_values(cuda, dtype, d):
+    """An infinite V gives an infinite result wherever its probability is not
+    0 -- exactly 1 (one key), 2^-6 or 2^-43 of the largest -- two of opposite
+    signs give NaN, and every other column is what it is without them."""
+    n, hq, s = 3, 4, 2000
+    q, k, v = torch.zeros(n, hq, 1, d), torch.zeros(n, 1, s, d), gen((n, 1, s, d), torch.float32, 81)
+    q[..., 0] = 1.0
+    k[:, 0, 37, 0], k[:, 0, 1500, 0] = -30.0, -4.0
+    lens = torch.tensor([s, 1800, 1], dtype=torch.int32)
+    v = v.to(dtype)
+    ref, _ = O.sdpa(npy(q[:2]), npy(k[:2, :, :1800]), npy(v[:2, :, :1800]), scale=1.0)
+    bad = v.clone()
+    bad[:, 0, 37, 3], bad[:, 0, 1500, 5], bad[:, 0, 40, 8] = math.inf, -math.inf, math.inf
+    bad[:, 0, 37, 9], bad[:, 0, 38, 9] = math.inf, -math.inf
+    bad[:, 0, 0, 11] = math.inf
+    lens[0] = 1800
+    out = npy(ops.sdpa_decode(q.to(dtype).to(cuda), k.to(dtype).to(cuda), bad.to(cuda), scale=1.0, kv_len=lens.to(cuda))[0])
+    for b in (0, 1):
+        assert np.isposinf(out[b, :, 0, [3, 8, 11]]).all() and np.isneginf(out[b, :, 0, 5]).all()
+        assert np.isnan(out[b, :, 0, 9]).all()
+        rest = [c for c in range(d) if c not in (3, 5, 8, 9, 11)]
+        close(torch.from_numpy(out[b][..., rest]), ref[b][..., rest])
+    assert np.isposinf(out[2, :, 0, 11]).all()
+    assert np.array_equal(np.delete(out[2, :, 0], 11, 1), np.tile(np.delete(npy(v[2, 0, 0]), 11), (hq, 1)))
 
 
 def test_sdpa_decode_shapes_share_workspace(cuda):
