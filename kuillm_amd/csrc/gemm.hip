@@ -31,6 +31,7 @@
 // test oracle, kuipy/kuiops.py:403-564, tests/test_jit_ops.py:51-112).
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "gemm_tile.hpp"
@@ -1376,6 +1377,10 @@ static int gemm_kernel_choice() {
     return choice;
 }
 
+// Work-groups of `threads` threads that one launch takes: a grid of 2^32 threads
+// along x and more wraps around, without an error.
+static int64_t max_groups(int threads) { return (((int64_t)1 << 32) - 1) / threads; }
+
 // Buffer offsets (tile rows x leading dim + K) must stay below 2^31 bytes.
 static bool offsets_fit(const GemmArgs &a, bool bcol) {
     const int64_t lim = (int64_t)1 << 30;
@@ -1464,10 +1469,11 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
         }
         return launch_status();
     }
-    const bool tile_ok = aligned && a.K > 0 && offsets_fit(a, bcol);
+    const TileCfg &t = kTiles[tc.tile];
+    const bool tile_ok = aligned && a.K > 0 && offsets_fit(a, bcol) &&
+                         cdiv(a.M, t.bm) * cdiv(a.N, t.bn) * batch <= max_groups(512);
     const int64_t t128 = cdiv(a.M, 128) * cdiv(a.N, 128) * batch;
-    const int bk = tile_ok ? kTiles[tc.tile].bk : 64, bm = tile_ok ? kTiles[tc.tile].bm : t128 < 2 * num_cus() ? 64 : 128,
-              bn = tile_ok ? kTiles[tc.tile].bn : 128;
+    const int bk = tile_ok ? t.bk : 64, bm = tile_ok ? t.bm : t128 < 2 * num_cus() ? 64 : 128, bn = tile_ok ? t.bn : 128;
     int splits = tile_ok ? tc.splits : (splits_req > 0 ? splits_req : max_s);
     if (batch != 1) splits = 1;
     a.tiles_m = (int)cdiv(a.M, bm);
@@ -1480,15 +1486,16 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
         if (!ws || ws_bytes < splits * part) return KUIOPS_E_WORKSPACE;
         a.partial = reinterpret_cast<float *>(ws);
     }
-    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
-    if (tile_ok && tiles * batch < INT32_MAX) {
+    if (tile_ok) {
         // vector stores: 16 bytes of the output, or of the fp32 partials
         if (splits > 1) a.vec_store = a.N % 4 == 0 && aligned16(ws);
         else if (sizeof(Tout) == 4) a.vec_store = a.ldo % 4 == 0 && a.stride_o % 4 == 0 && aligned16(a.out);
         else a.vec_store = a.N % 8 == 0 && a.ldo % 8 == 0 && a.stride_o % 8 == 0 && aligned16(a.out);
-        const dim3 grid((unsigned)(tiles * batch), (unsigned)splits);
+        const dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n * batch), (unsigned)splits);
         if (splits > 1) launch_tile<T, Tout, true>(tc.tile, a, bcol, grid, st);
         else launch_tile<T, Tout, false>(tc.tile, a, bcol, grid, st);
+    } else if ((int64_t)a.tiles_m * a.tiles_n > max_groups(256)) {
+        return KUIOPS_E_UNSUPPORTED;
     } else if (splits > 1) {
         launch_mfma<T, Tout, true>(bm, a, bcol, splits, st);
     } else {
@@ -1504,8 +1511,27 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
 // of 4 while one work-group per CU runs (1 x 4096 x 4096 48 -> 41).
 static int run_f32(GemmArgs a, int64_t batch, bool bcol, hipStream_t st) {
     const bool big = a.M > 32 && cdiv(a.M, 64) * cdiv(a.N, 64) * batch >= num_cus();
-    const int64_t tm = cdiv(a.M, big ? 64 : 32), tn = cdiv(a.N, big ? 64 : 32);
-    if (tm * tn * batch > INT32_MAX) return KUIOPS_E_UNSUPPORTED;
+    const int64_t bt = big ? 64 : 32, tm = cdiv(a.M, bt), tn = cdiv(a.N, bt), most = max_groups(256);
+    if (tm * tn * batch > most) {
+        // more tiles than one launch takes: whole products a launch, or rows of one
+        const int64_t nb = std::min(batch, std::max<int64_t>(1, most / (tm * tn)));
+        const int64_t rows = nb > 1 || tm * tn <= most ? a.M : most / tn * bt;
+        const float *A = reinterpret_cast<const float *>(a.A), *B = reinterpret_cast<const float *>(a.B);
+        const float *cin = reinterpret_cast<const float *>(a.cin);
+        float *out = reinterpret_cast<float *>(a.out);
+        for (int64_t b = 0; b < batch; b += nb)
+            for (int64_t m = 0; m < a.M; m += rows) {
+                GemmArgs p = a;
+                p.A = A + b * a.stride_a + m * a.lda;
+                p.B = B + b * a.stride_b;
+                p.out = out + b * a.stride_o + m * a.ldo;
+                if (a.c_kind == KUIOPS_C_FULL) p.cin = cin + m * a.ldcin;
+                p.M = std::min(rows, a.M - m);
+                const int s = run_f32(p, std::min(nb, batch - b), bcol, st);
+                if (s != KUIOPS_OK) return s;
+            }
+        return KUIOPS_OK;
+    }
     a.tiles_m = (int)tm;
     a.tiles_n = (int)tn;
     const dim3 grid((unsigned)(tm * tn * batch)), block(256);

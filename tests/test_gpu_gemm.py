@@ -209,6 +209,21 @@ def test_mm_f32_tiles(cuda, layout, M, N, K):
     assert ((batch[2].cpu().double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("dtype, K, N", [(torch.float32, 4, 8224), (torch.bfloat16, 8, 33024)])
+def test_bmm_more_tiles_than_a_launch(cuda, dtype, K, N):
+    """65535 products of one row: 2^24 fp32 tiles of 32 columns, 2^23 bf16 ones
+    of 256 (a launch of 2^32 threads along x wraps around).  One B for all;
+    small whole numbers, so the results are exact."""
+    batch = 65535
+    g = torch.Generator(device=cuda).manual_seed(3)
+    A = torch.randint(-3, 4, (batch, 1, K), device=cuda, generator=g).to(dtype)
+    B = torch.randint(-3, 4, (K, N), device=cuda, generator=g).to(dtype)
+    out = ops.bmm(A, B.expand(batch, -1, -1))
+    for rows in range(0, batch, 4096):
+        want = A[rows:rows + 4096, 0].float() @ B.float()
+        assert torch.equal(out[rows:rows + 4096, 0].float(), want), rows
+
+
 def test_mm_rows_past_buffer_offsets(cuda):
     """A row-major B whose rows lie 32 MiB apart (offsets past 2^31 bytes)."""
     M, N, K, ld = 130, 64, 72, 1 << 24
