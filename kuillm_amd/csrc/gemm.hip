@@ -1345,7 +1345,7 @@ static void launch_tile(int tile, const GemmArgs &a, bool bcol, dim3 grid, hipSt
 
 template <typename Tout>
 static void launch_reduce(const GemmArgs &a, hipStream_t st) {
-    const bool vec = a.N % 4 == 0 && a.ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(a.out) & (4 * sizeof(Tout) - 1)) == 0;
+    const bool vec = a.N % 4 == 0 && a.ldo % 4 == 0 && aligned16(a.partial) && (reinterpret_cast<uintptr_t>(a.out) & (4 * sizeof(Tout) - 1)) == 0;
     const int64_t by = cdiv(a.M, 4);
     const dim3 grid((unsigned)cdiv(a.N, vec ? 256 : 64), (unsigned)(by < 65535 ? by : 65535));
     if (vec) hipLaunchKernelGGL((splitk_reduce_kernel<Tout, true>), grid, dim3(256), 0, st, a);
@@ -1429,7 +1429,7 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
         if (aligned && !any_ws) return KUIOPS_E_WORKSPACE;
         // (unaligned operands, and the decode GEMM, split as far as the
         // workspace they were given allows)
-        max_s = ws && part > 0 ? (int)min((int64_t)max_s, (int64_t)(ws_bytes / part)) : 1;
+        max_s = ws_ok && part > 0 ? (int)min((int64_t)max_s, (int64_t)(ws_bytes / part)) : 1;
         if (max_s < 1) max_s = 1;
     }
     const TileChoice tc = choose_tile(a.M, a.N, a.K, batch, ws_ok ? max_s : 1,
@@ -1476,6 +1476,12 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
     const int bk = tile_ok ? t.bk : 64, bm = tile_ok ? t.bm : t128 < 2 * num_cus() ? 64 : 128, bn = tile_ok ? t.bn : 128;
     int splits = tile_ok ? tc.splits : (splits_req > 0 ? splits_req : max_s);
     if (batch != 1) splits = 1;
+    // Unaligned operands need no workspace, whatever split count is asked for,
+    // and take as many splits as it allows up to max_splits: a stage waits for
+    // its loads, so shorter K ranges pay (us with 1, 2, 4 and all splits:
+    // 4 x 4095 x 4095 62 / 38 / 25 / 17, 300 x 1001 x 2047 40 / 28 / 23 / 23,
+    // 777 x 777 x 1555 33 / 25 / - / 23; 500 x 2049 x 5633 93 / 57 / 50 / 49, 45 with 3).
+    if (!aligned && splits > 1) splits = ws_ok ? (int)max((int64_t)1, min((int64_t)splits, (int64_t)(ws_bytes / part))) : 1;
     a.tiles_m = (int)cdiv(a.M, bm);
     a.tiles_n = (int)cdiv(a.N, bn);
     const int64_t kps = cdiv(cdiv(a.K, splits), bk) * bk;

@@ -209,6 +209,31 @@ def test_mm_f32_tiles(cuda, layout, M, N, K):
     assert ((batch[2].cpu().double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("K, splits, offset, ok", [
+    (1031, 0, None, True), (1031, 3, None, True), (1031, 3, 0, True), (1031, 40, 0, True), (1031, 3, 2, True),
+    (1032, 3, 0, True), (1032, 3, 4, True), (1032, 3, None, False)])
+def test_addmm_split_requests(cuda, K, splits, offset, ok):
+    """kuiops_addmm with a split count of the caller's: operands of odd length
+    take any workspace or none (splits as it allows), aligned ones need it; one
+    at another alignment than 16 bytes is as good.  Whole numbers: exact."""
+    M, N = 70, 132
+    g = torch.Generator().manual_seed(4)
+    A, B = (torch.randint(-2, 3, s, generator=g).to(torch.bfloat16).to(cuda) for s in ((M, K), (N, K)))
+    out = torch.full((M, N), float("nan"), device=cuda)
+    # three splits' partials (40 do not fit)
+    store = torch.empty(3 * M * N * 4 + 64, dtype=torch.uint8, device=cuda)
+    ws = None if offset is None else store[offset:]
+    lib = _lib.load()
+    status = lib.kuiops_addmm(M, K, N, 1.0, 0.0, _lib.BF16, A.data_ptr(), K, B.data_ptr(), K, _lib.B_COL, None,
+                              _lib.C_NONE, 0, _lib.F32, out.data_ptr(), N, splits, None if ws is None else ws.data_ptr(),
+                              0 if ws is None else ws.numel(), torch.cuda.current_stream().cuda_stream)
+    if not ok:
+        assert status == _lib.E_WORKSPACE
+        return
+    assert status == _lib.OK
+    assert torch.equal(out, A.float() @ B.float().t())
+
+
 @pytest.mark.parametrize("dtype, K, N", [(torch.float32, 4, 8224), (torch.bfloat16, 8, 33024)])
 def test_bmm_more_tiles_than_a_launch(cuda, dtype, K, N):
     """65535 products of one row: 2^24 fp32 tiles of 32 columns, 2^23 bf16 ones
