@@ -49,7 +49,8 @@ def _stream(dev: torch.device) -> int:
 
 @functools.lru_cache(maxsize=4096)
 def _query_workspace(op: int, a: int, b: int, c: int) -> int:
-    """kuiops_query_workspace: a function of its arguments alone."""
+    """kuiops_query_workspace for the ops whose size follows from the arguments
+    alone (decode_rows_batched's splits also follow the device's CUs)."""
     return _lib_handle().kuiops_query_workspace(op, a, b, c)
 
 
@@ -1185,7 +1186,7 @@ def decode_rows_batched(x, W, x_kind="plain", out_kind="plain", in_add=None, nor
     elif out_kind == "swiglu":
         pair_off = N // 2
     lib = _lib_handle()
-    ws_bytes = _query_workspace(_lib.OP_DECODE_ROWS_BATCHED, M, N, K) if split else 0
+    ws_bytes = lib.kuiops_query_workspace(_lib.OP_DECODE_ROWS_BATCHED, M, N, K) if split else 0
     ws = workspace(x.device, ws_bytes, "decode_rows") if ws_bytes else None
     _lib.check("kuiops_decode_rows_batched", lib.kuiops_decode_rows_batched(
         M, N, K, _dt(x.dtype), _X_KIND[x_kind], _OUT_KIND[out_kind], x.data_ptr(), x.stride(0), _ptr(row), rows,

@@ -223,3 +223,30 @@ def test_rmsnorm_refuses_overlapping_rows(lib):
     for ldr, ldro in ((32, None), (-64, None), (None, 32), (None, 0), (64, 32)):
         assert call(4, ldr, ldro) == _lib.E_INVALID
         assert call(0, ldr, ldro) == _lib.OK
+
+
+def test_decode_rows_workspace_follows_the_device(monkeypatch):
+    """decode_rows_batched's workspace depends on the current device's CUs, so
+    its size is asked for on every call."""
+    import torch
+
+    from kuillm_amd import ops
+
+    class Lib:
+        sizes, given = [4096, 8192], []
+
+        def kuiops_query_workspace(self, op, a, b, c):
+            return self.sizes[len(self.given)]
+
+        def kuiops_decode_rows_batched(self, *args):
+            self.given.append(args[-2])
+            return _lib.OK
+
+    lib = Lib()
+    monkeypatch.setattr(ops, "_lib_handle", lambda: lib)
+    monkeypatch.setattr(ops, "_stream", lambda dev: 0)
+    monkeypatch.setattr(ops, "workspace", lambda dev, size, kind="": torch.empty(size, dtype=torch.uint8))
+    x, W = torch.zeros(2, 64, dtype=torch.bfloat16), torch.zeros(16, 64, dtype=torch.bfloat16)
+    for _ in lib.sizes:
+        ops.decode_rows_batched(x, W)
+    assert lib.given == lib.sizes
