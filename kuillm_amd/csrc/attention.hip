@@ -894,12 +894,14 @@ static int64_t decode_chunk(int64_t s) {
 
 // Query rows per work-group (of the rows sharing a KV head): 16 on the MFMA
 // kernel, which takes 3 or more rows (with one or two its MFMAs are mostly
-// empty and the VALU form has little to do) and key rows whose byte offsets
-// fit 31 bits; else up to 8.
+// empty and the VALU form has little to do), key rows whose byte offsets fit 31
+// bits and V rows that do not overlap (its V descriptor ends at the last key, so
+// past it a row that begins earlier, as in an expanded V, would still be read);
+// else up to 8.
 constexpr int kMfmaRows = 16;
-static int decode_rows_per_group(int64_t s, int rows_kv, int64_t sk2, int64_t sv2) {
+static int decode_rows_per_group(int64_t s, int64_t hd, int rows_kv, int64_t sk2, int64_t sv2) {
     const int64_t st = sk2 > sv2 ? sk2 : sv2;
-    if (rows_kv >= 3 && s < (1 << 30) && sk2 >= 0 && sv2 >= 0 && (s + 64) * st * 2 < ((int64_t)1 << 31)) return kMfmaRows;
+    if (rows_kv >= 3 && s < (1 << 30) && sk2 >= 0 && sv2 >= hd && (s + 64) * st * 2 < ((int64_t)1 << 31)) return kMfmaRows;
     return rows_kv <= 1 ? 1 : rows_kv <= 2 ? 2 : rows_kv <= 4 ? 4 : 8;
 }
 
@@ -1009,7 +1011,7 @@ static int launch_decode(AttnArgs a, hipStream_t st) {
                            dim3(kDecodeWideWaves * 64), 0, st, a);
         return launch_status();
     }
-    const int R = decode_rows_per_group(a.s, rows_kv, a.sk2, a.sv2);
+    const int R = decode_rows_per_group(a.s, HD, rows_kv, a.sk2, a.sv2);
     a.rows_per_group = R;
     a.row_groups = (int)cdiv(rows_kv, R);
     dim3 grid((unsigned)a.splits, (unsigned)(a.hkv * a.row_groups), (unsigned)a.n);
@@ -1023,14 +1025,15 @@ static int launch_decode(AttnArgs a, hipStream_t st) {
     }
     if (a.splits == 1) {
         // short caches: one work-group per row group streams every key (no
-        // workspace round trip).  Four rows take 4-wave work-groups: at 180
-        // VGPRs two of them fit a CU, so batch 64's 512 row groups run in one
-        // round instead of two 8-wave rounds (27 -> ~22 us per layer).
+        // workspace round trip).  Four and eight rows (caches that the MFMA
+        // kernel does not take) have 4-wave work-groups: at 180 VGPRs two of
+        // them fit a CU, so 512 row groups run in one round instead of two
+        // 8-wave rounds (64 sequences, 8 KV heads of 64, 640 keys: 27 -> 22 us).
         switch (R) {
             case 1: hipLaunchKernelGGL((fa_decode_kernel<T, HD, 1, 16>), grid, dim3(1024), 0, st, a); break;
             case 2: hipLaunchKernelGGL((fa_decode_kernel<T, HD, 2, 16>), grid, dim3(1024), 0, st, a); break;
-            // (query first: the early K / V loads cost this instance 24 VGPRs
-            // and measured 1.697 against 1.683 ms per batch-64 step)
+            // (query first: the early K / V loads cost this instance 24 VGPRs,
+            // 1.697 against 1.683 ms for the whole decode step of those 64)
             case 4: hipLaunchKernelGGL((fa_decode_kernel<T, HD, 4, 4, 4, false>), grid, dim3(256), 0, st, a); break;
             default: hipLaunchKernelGGL((fa_decode_kernel<T, HD, 8, 4>), grid, dim3(256), 0, st, a); break;
         }
@@ -1122,7 +1125,7 @@ extern "C" int kuiops_sdpa_decode(int64_t n, int64_t hq, int64_t hkv, int64_t l,
     fill_args(a, n, hq, hkv, l, s, Q, sq, K, sk, V, sv, O, so, lse, scale, causal);
     a.kv_len = kv_len;
     const int64_t ss = s > 0 ? s : 1;
-    const int R = decode_rows_per_group(s, (int)((hq / hkv) * l), a.sk2, a.sv2);
+    const int R = decode_rows_per_group(s, ev, (int)((hq / hkv) * l), a.sk2, a.sv2);
     a.chunk = decode_chunk_for(ss, n * hkv * cdiv((hq / hkv) * l, R), R == kMfmaRows ? 1 : 2);
     if (decode_row_wide(ss, ev, n * hq * l) || decode_single_split(ss, ev, R)) a.chunk = ss;
     a.splits = (int)cdiv(ss, a.chunk);

@@ -188,7 +188,7 @@ DECODE = [  # n, hq, hkv, l, s, d
     (1, 16, 4, 1, 384, 128),    # row-wide at head dim 128 (longest)
     (2, 8, 2, 1, 77, 128),
     (1, 4, 4, 1, 1, 64),
-    (64, 32, 8, 1, 300, 64),    # 512 row groups of 4 rows: one split, 4-wave work-groups
+    (64, 32, 8, 1, 300, 64),    # 512 row groups: one split
     (70, 32, 8, 1, 520, 64),
 ]
 
@@ -300,6 +300,39 @@ def test_sdpa_decode_infinite_values(cuda, dtype, d):
         close(torch.from_numpy(out[b][..., rest]), ref[b][..., rest])
     assert np.isposinf(out[2, :, 0, 11]).all()
     assert np.array_equal(np.delete(out[2, :, 0], 11, 1), np.tile(np.delete(npy(v[2, 0, 0]), 11), (hq, 1)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,hq,hkv,l,s,d", [
+    # 4 rows per work-group: 32 splits (merged by a second kernel), 16 and 2 (in the kernel), one
+    (2, 8, 2, 1, 2000, 64), (16, 6, 2, 1, 3000, 128), (160, 4, 2, 2, 301, 64), (260, 8, 2, 1, 301, 128),
+    # 8 rows: 32 splits, 15 of three row groups, 16, one
+    (2, 16, 2, 1, 2000, 128), (3, 40, 2, 1, 900, 64), (16, 10, 2, 1, 3000, 64), (260, 12, 2, 1, 301, 128)])
+def test_sdpa_decode_overlapping_values(cuda, dtype, n, hq, hkv, l, s, d):
+    """Three and more rows per KV head where V's rows overlap, which is the
+    vector kernels' work: rows 8 elements apart with NaN from the first one
+    that only keys past the sequence's count hold, and one row expanded over
+    all keys, infinite in one column.  |error| <= half an ulp of the result."""
+    q, k = gen((n, hq, l, d), dtype, 91), gen((n, hkv, s, d), dtype, 92)
+    store = gen((n, hkv, 8 * s + d), dtype, 93)
+    lens = torch.randint(l, s + 1, (n,), generator=torch.Generator().manual_seed(s), dtype=torch.int32)
+    lens[0] = s - 1
+    for b, m in enumerate(lens.tolist()):
+        store[b, :, 8 * (m - 1) + d:] = math.nan
+    v = store.to(cuda).as_strided((n, hkv, s, d), (hkv * (8 * s + d), 8 * s + d, 8, 1))
+    qd, kd, ld = q.to(cuda), k.to(cuda), lens.to(cuda)
+    out, lse = ops.sdpa_decode(qd, kd, v, return_lse=True, kv_len=ld)
+    one = gen((n, hkv, 1, d), dtype, 94)
+    one[:, :, :, 5] = math.inf
+    same, _ = ops.sdpa_decode(qd, kd, one.to(cuda).expand(n, hkv, s, d), causal=False, kv_len=ld)
+    rows = one.repeat_interleave(hq // hkv, 1).expand(n, hq, l, d)
+    assert torch.isposinf(same[..., 5]).all()
+    close(torch.cat([same[..., :5], same[..., 6:]], -1), npy(torch.cat([rows[..., :5], rows[..., 6:]], -1)))
+    for b in (0, 1, n - 1):
+        m = int(lens[b])
+        ref, lref = O.sdpa(npy(q[b:b + 1]), npy(k[b:b + 1, :, :m]), npy(v[b:b + 1, :, :m]), causal=True, align="bottom_right")
+        close(out[b:b + 1], ref)
+        np.testing.assert_allclose(npy(lse[b:b + 1]), lref, atol=1e-3, rtol=1e-4)
 
 
 def test_sdpa_decode_shapes_share_workspace(cuda):
