@@ -1045,10 +1045,16 @@ extern "C" int kuiops_rope_kv_append(int64_t n, int64_t t, int64_t hq, int64_t h
                q_out, sq[0], sq[1], sq[2], k_cache, sk[0], sk[1], sk[2], v_cache, sv[0], sv[1], sv[2], cache_cap};
     const dim3 grid((unsigned)t, (unsigned)n, (unsigned)(hq + 2 * hkv));
     hipStream_t st = as_stream(stream);
-    // one work-group per token from 128 tokens (fewer spread over more CUs by
-    // head: 64 tokens 2.7 us by head, 2.95 by token; 512: 7.6 and 3.4)
+    // One work-group per token where the heads make more one-wave work-groups than
+    // the CUs take in a round or two (us by head and by token, head dim 64: 64
+    // tokens of 32 + 8 heads 2.7 / 2.95, 200 3.2 / 2.9 with 12 + 4, 512 7.6 / 3.4
+    // with 32 + 8; 4 + 1 heads: 400 tokens 2.7 / 2.9, 1000 3.6 / 3.0; 1 + 1 heads:
+    // 400 2.4 / 3.0, 4000 4.6 / 5.1), and tokens enough for their rows (head dim 256,
+    // 32 + 8 heads: 128 tokens 4.5 / 4.8, 200 5.8 / 5.4).
+    const int64_t heads = hq + 2 * hkv;
+    const bool by_token = n * t >= (hd > 128 ? 192 : 128) && heads >= 4 && n * t * heads >= 3000;
     const auto aligned8 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
-    if (n * t >= 128 && hd / 2 <= kRopeMaxHalf && !(sq[0] % 4 || sq[1] % 4 || sq[2] % 4 || sk[0] % 4 || sk[1] % 4 || sk[2] % 4) &&
+    if (by_token && hd / 2 <= kRopeMaxHalf && !(sq[0] % 4 || sq[1] % 4 || sq[2] % 4 || sk[0] % 4 || sk[1] % 4 || sk[2] % 4) &&
         aligned8(q_out) && aligned8(k_cache)) {
         const dim3 g((unsigned)t, (unsigned)n);
         if (dtype == KUIOPS_BF16) hipLaunchKernelGGL((rope_kv_token_kernel<bf16_t>), g, dim3(256), 0, st, a);

@@ -60,7 +60,10 @@ def test_silu_mul_vs_oracle(cuda, m, n):
 
 
 @pytest.mark.parametrize("n,t,hq,hkv,hd,p0", [(1, 1, 32, 8, 64, 517), (2, 9, 4, 2, 128, 3), (1, 40, 8, 8, 64, 0),
-                                                  (3, 43, 5, 1, 72, 2), (1, 128, 32, 8, 128, 90)])    # one work-group per token
+                                                  (3, 43, 5, 1, 72, 2),
+                                                  # one work-group per token: enough tokens and heads, at the lines
+                                                  (1, 128, 32, 8, 128, 90), (3, 200, 5, 1, 72, 2), (2, 375, 2, 1, 64, 0),
+                                                  (1, 192, 14, 1, 256, 7)])
 def test_rope_kv_append_vs_oracle(cuda, n, t, hq, hkv, hd, p0):
     cap = p0 + t + 5
     qkv = bf((n, t, (hq + 2 * hkv) * hd), 5)
