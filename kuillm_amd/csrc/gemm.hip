@@ -1514,7 +1514,17 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
 // 64x64 tiles where they give every CU a work-group, else 32x32 (us, 64x64
 // against 32x32: 512 x 2048 x 2048 58 / 61, 2048^3 175 / 228, 200 x 3000 x 1003
 // 42 / 31, 19 x 16256 x 5056 184 / 83), whose K is split over 8 waves instead
-// of 4 while one work-group per CU runs (1 x 4096 x 4096 48 -> 41).
+// of 4 while one work-group per CU runs (1 x 4096 x 4096 48 -> 41), and over no
+// more waves than a short K has stages of 32 for: the others' loads, LDS and sums
+// are for nothing, and fewer work-groups fit a CU (us with 1, 2, 4, 8 waves: 1 x
+// 432 x 32 4.1 / 4.4 / 4.9 / 6.1, 200 x 3001 x 24 5.2 / 6.2 / 10.0 / 17.5, x 64 6.7 /
+// 6.0 / 9.9 / 17.4, x 128 11.1 / 8.0 / 9.9 / 17.4; 1 x 432 x 100 9.0 / 5.8 / 4.8 / 6.0).
+template <int WK>
+static void launch_f32_small(const GemmArgs &a, bool bcol, dim3 grid, hipStream_t st) {
+    if (bcol) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, WK, true>), grid, dim3(WK * 64), 0, st, a);
+    else hipLaunchKernelGGL((gemm_f32_kernel<1, 1, WK, false>), grid, dim3(WK * 64), 0, st, a);
+}
+
 static int run_f32(GemmArgs a, int64_t batch, bool bcol, hipStream_t st) {
     const bool big = a.M > 32 && cdiv(a.M, 64) * cdiv(a.N, 64) * batch >= num_cus();
     const int64_t bt = big ? 64 : 32, tm = cdiv(a.M, bt), tn = cdiv(a.N, bt), most = max_groups(256);
@@ -1543,10 +1553,10 @@ static int run_f32(GemmArgs a, int64_t batch, bool bcol, hipStream_t st) {
     const dim3 grid((unsigned)(tm * tn * batch)), block(256);
     if (big && bcol) hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 1, true>), grid, block, 0, st, a);
     else if (big) hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 1, false>), grid, block, 0, st, a);
-    else if (tm * tn * batch <= num_cus() && bcol) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 8, true>), grid, dim3(512), 0, st, a);
-    else if (tm * tn * batch <= num_cus()) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 8, false>), grid, dim3(512), 0, st, a);
-    else if (bcol) hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 4, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((gemm_f32_kernel<1, 1, 4, false>), grid, block, 0, st, a);
+    else if (a.K <= 32) launch_f32_small<1>(a, bcol, grid, st);
+    else if (a.K <= 64) launch_f32_small<2>(a, bcol, grid, st);
+    else if (a.K <= 128 || tm * tn * batch > num_cus()) launch_f32_small<4>(a, bcol, grid, st);
+    else launch_f32_small<8>(a, bcol, grid, st);
     return launch_status();
 }
 

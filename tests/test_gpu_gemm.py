@@ -184,9 +184,10 @@ def test_bmm_odd_strides(cuda, dtype, b, M, K, N, layout):
 
 
 @pytest.mark.parametrize("layout", ["row", "col"])
-@pytest.mark.parametrize("M,N,K", [(1, 4096, 96), (33, 31, 257), (64, 3072, 768), (300, 1000, 1003), (1000, 1030, 130), (7, 9000, 5)])
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 96), (33, 31, 257), (64, 3072, 768), (300, 1000, 1003), (1000, 1030, 130), (7, 9000, 5),
+                                   (1, 1, 1), (40, 33, 31), (35, 500, 32), (33, 70, 33), (5, 3000, 64), (100, 31, 65), (31, 9000, 128), (66, 40, 129)])
 def test_mm_f32_tiles(cuda, layout, M, N, K):
-    """fp32 MFMA tiles (32x32 with 8 and 4 K slices, 64x64), ragged in every
+    """fp32 MFMA tiles (32x32 with 1, 2, 4 and 8 K slices, 64x64), ragged in every
     size, operands inside NaN-filled storage, against a 64-bit product:
     fp32 sums of K products of size s are within K * 2^-24 * sum|s|, here
     taken as the root-mean-square bound 2^-24 * K relative to the row norms."""
