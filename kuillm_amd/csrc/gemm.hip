@@ -24,8 +24,8 @@
 // same XCD (dispatch is round-robin over the 8 XCDs, each with its own L2)
 // and are visited in groups of 8 tile-rows.
 //
-// f32: `gemm_f32_kernel`, fp32 MFMAs.  f64: `gemm_simt_kernel`, a plain
-// LDS-tiled kernel with the same epilogue.
+// f32: `gemm_f32_kernel`, fp32 MFMAs.  f64, and odd strides with a short K:
+// `gemm_simt_kernel`, a plain LDS-tiled kernel with the same epilogue.
 //
 // Semantics follow aten mm / addmm / bmm (the reference's fallthrough and
 // test oracle, kuipy/kuiops.py:403-564, tests/test_jit_ops.py:51-112).
@@ -1211,7 +1211,8 @@ __global__ __launch_bounds__(WM * WN * WK * 64) void gemm_f32_kernel(GemmArgs a)
     store_tile32<float>(a, acc, m0 + wm * 32, n0 + wn * 32 + lr, h);
 }
 
-// LDS-tiled SIMT GEMM (fp64; any strides and shapes): 64x64 tile, 256 threads each owning a 4x4 strided patch, K step 16.
+// LDS-tiled SIMT GEMM (fp64, and 16-bit operands of odd strides with a short K:
+// simt_faster): 64x64 tile, 256 threads each owning a 4x4 strided patch, K step 16.
 template <typename Tin, typename Tacc, typename Tout>
 __global__ __launch_bounds__(256) void gemm_simt_kernel(GemmArgs a, int b_col) {
     __shared__ Tacc sA[16][65];
@@ -1575,6 +1576,22 @@ static bool rows_aligned(const GemmArgs &a, bool bcol, int64_t batch) {
     return bcol || a.N % 8 == 0;
 }
 
+// 16-bit operands of odd strides whose K is so short that gemm_mfma_kernel's time
+// is its stage of 64 k, not its arithmetic: up to K = 16 always (its K tail is
+// loaded by elements), up to 32 for few tiles or ones that are mostly empty (and
+// the transposing of a row-major B is in vain), up to 48 for many of those (us,
+// SIMT against MFMA, row-major B: 9 x (5 x 59) K = 7 4.0 / 6.3, K = 21 5.8 / 6.2, K =
+// 41 7.6 / 6.1; 100 x (1 x 511) K = 25 9.3 / 11.4, K = 37 11.6 / 11.5; 209 x (496 x 23) K
+// = 7 10.1 / 22.3, K = 41 19.6 / 22.5, K = 64 24.5 / 20.0; 3000 x 5001 K = 8 21.5 /
+// 21.7, K = 31 34.2 / 29.4).
+static bool simt_faster(const GemmArgs &a, int64_t batch, bool bcol) {
+    if (cdiv(a.M, 64) > 65535 * 32 || cdiv(a.N, 64) > 65535) return false;
+    const int64_t tiles = cdiv(a.M, 64) * cdiv(a.N, 128) * batch;
+    const bool empty = a.N <= 32 && tiles > 2 * num_cus();
+    if (a.K > 32) return a.K <= 48 && empty && !bcol;
+    return a.K <= 16 || tiles <= 128 || empty || (!bcol && (a.N <= 64 || a.M <= 16));
+}
+
 // Shared entry for mm / addmm / bmm.
 static int gemm_entry(GemmArgs a, int64_t batch, int in_dt, int out_dt, int b_layout, int splits,
                       void *ws, size_t ws_bytes, void *stream) {
@@ -1589,6 +1606,12 @@ static int gemm_entry(GemmArgs a, int64_t batch, int in_dt, int out_dt, int b_la
     if (in_dt == KUIOPS_BF16 || in_dt == KUIOPS_F16) {
         if (a.M > INT32_MAX / 2 || a.N > INT32_MAX / 2) return KUIOPS_E_UNSUPPORTED;
         const bool al = rows_aligned(a, bcol, batch);
+        if (!al && splits <= 1 && simt_faster(a, batch, bcol)) {
+            if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_BF16) return run_simt<bf16_t, float, bf16_t>(a, batch, bcol, st);
+            if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_F32) return run_simt<bf16_t, float, float>(a, batch, bcol, st);
+            if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F16) return run_simt<f16_t, float, f16_t>(a, batch, bcol, st);
+            if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F32) return run_simt<f16_t, float, float>(a, batch, bcol, st);
+        }
         if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_BF16) return run_mfma<bf16_t, bf16_t>(a, batch, bcol, al, splits, ws, ws_bytes, st);
         if (in_dt == KUIOPS_BF16 && out_dt == KUIOPS_F32) return run_mfma<bf16_t, float>(a, batch, bcol, al, splits, ws, ws_bytes, st);
         if (in_dt == KUIOPS_F16 && out_dt == KUIOPS_F16) return run_mfma<f16_t, f16_t>(a, batch, bcol, al, splits, ws, ws_bytes, st);

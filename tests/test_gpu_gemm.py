@@ -165,7 +165,12 @@ def test_addmm_tile_kernel_edges(cuda, layout, M, N, K):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("b,M,K,N", [(5, 77, 77, 64), (3, 130, 201, 131), (2, 1, 7, 9), (4, 333, 129, 128), (1, 257, 1031, 255),
-                                     (45, 500, 67, 260)])      # 128x128 tiles; the others 64x128
+                                     (45, 500, 67, 260),       # 128x128 tiles; the others 64x128
+                                     # short K: the vector kernel up to 16, 32 (few tiles) and 48 (few columns, many tiles)
+                                     (3, 65, 16, 63), (2, 130, 15, 257), (32, 70, 32, 129), (300, 65, 48, 32), (260, 129, 47, 31),
+                                     (200, 16, 31, 130), (160, 70, 29, 63),
+                                     # one past each line
+                                     (260, 65, 17, 130), (2, 70, 33, 129), (300, 65, 49, 31), (300, 65, 47, 33), (33, 70, 31, 129)])
 @pytest.mark.parametrize("layout", ["row", "col"])
 def test_bmm_odd_strides(cuda, dtype, b, M, K, N, layout):
     """Rows of odd length at 2-byte alignment: slices of wider NaN-filled
