@@ -1305,13 +1305,18 @@ struct TileChoice { int tile, splits; float us; };
 
 // The tile and split count of least estimated time: rounds of one tile per
 // CU, and for a split the partials' traffic plus the second launch.  max_s
-// bounds the splits; fixed_s > 0 asks for that many.
+// bounds the splits; fixed_s > 0 asks for that many.  Up to 64 columns in more
+// 64x64 tiles than CUs, those are always fastest: two and more fit a CU, which the
+// model does not count, and larger ones share nothing (209 x (496 x 24), us for 64x64
+// / 128x64 / 128x128: K = 64 12.7 / 18.4 / 16.6, K = 512 30.4 / 35.7 / 35.6; 60000 x 64,
+// K = 128 9.3 / 11.0 / 10.9).
 static TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int max_s, int fixed_s) {
     TileChoice best{0, 1, 1e30f};
     const int64_t cus = num_cus();
     for (int t = 0; t < kNumTiles; ++t) {
         const TileCfg &c = kTiles[t];
         const int64_t tiles = cdiv(M, c.bm) * cdiv(N, c.bn) * batch;
+        if (t > 0 && N <= 64 && cdiv(M, 64) * batch > cus) break;
         for (int s = fixed_s > 0 ? fixed_s : 1; s <= (fixed_s > 0 ? fixed_s : max_s); ++s) {
             const int64_t rounds = cdiv(tiles * s, cus);
             const int64_t stages = cdiv(cdiv(K, s), c.bk);
