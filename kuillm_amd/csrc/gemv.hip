@@ -11,9 +11,9 @@
 //     W operand); the waves' K ranges are summed in LDS in wave order.
 //   * gemm_tile_kernel (gemm_tile.hpp; K-contiguous W, i.e. an nn.Linear weight
 //     seen through .t(), and a row-major W too narrow for the kernels above to
-//     fill the CUs: tiles_faster).
-//   * gemv_splitk_kernel (a caller's own split count, fp32 outputs with a bias):
-//     one 16-byte load per lane is already an MFMA operand; `splits`
+//     fill the CUs, or more than 16 rows: tiles_faster).
+//   * gemv_splitk_kernel (a short K, a caller's own split count, fp32 outputs with
+//     a bias): one 16-byte load per lane is already an MFMA operand; `splits`
 //     work-groups share a strip and gemv_reduce_kernel sums their partials in
 //     split order.
 //
@@ -705,21 +705,42 @@ static bool rows_eligible(const GemvArgs &a, bool wcol) {
     return true;
 }
 
-// Products that the MFMA tile kernel streams faster than the kernels here: every
-// K-contiguous W, whose 16 lanes x 16 bytes of a k step read 64-byte pieces of
-// 16 rows (gemv_splitk_kernel; us for M = 1 / 16 / 64, against the tile kernel:
-// 4096 x 4096 16.6 / 16.9 / 29.4 -> 11.0 / 11.5 / 13.2, 32000 x 2048 38 / 41 / 74
-// -> 32 / 32 / 33.5, 2048 x 5632 20.5 / 23.4 / 37 -> 9.9 / 10.3 / 11.9), and a
-// row-major W unless its strips or column blocks fill the CUs and x is short
-// (11008 x 4096, M = 1 / 16 / 64: 18.1 / 23.0 / 34.3 here, 22.2 / 21.5 / 26.3 there;
-// 2048 x 5632: 11.6 / 15.6 / 30.2 and 9.9 / 10.5 / 12.3).
 int gemm_decode_tiles(int64_t M, int64_t N, int64_t K, int in_dt, const void *x, int64_t ldx, const void *W,
                       int64_t ldw, bool wcol, const void *bias, int out_dt, void *out, int64_t ldo, void *ws,
                       size_t ws_bytes, hipStream_t st);
 
-static bool tiles_faster(int64_t M, int64_t N, int64_t K, bool wcol) {
+// Products that the MFMA tile kernel streams faster than the kernels here
+// (weights cold in HBM; us here against there).
+//   * Up to 16 rows and K = 128 are no work for its pipeline: 5 x 3704, K = 8 /
+//     64 / 128 / 160, 3.1 / 3.1 / 3.3 / 5.4 against 3.6 / 3.6 / 3.8 / 3.6; a K-contiguous
+//     W is level at K = 128 (3.6), but 4.3 / 5.3 with more than a tile per CU (20000
+//     columns); gemv_rows_kernel with 512 columns (1 x 512 of K = 64, 3.1 / 3.5).
+//   * Every other K-contiguous W goes there: its 16 lanes x 16 bytes of a k step read
+//     64-byte pieces of 16 rows (gemv_splitk_kernel; M = 1 / 16 / 64: 4096 x 4096 16.6 /
+//     16.9 / 29.4 against 11.0 / 11.5 / 13.2, 2048 x 5632 20.5 / 23.4 / 37 against 9.9 /
+//     10.3 / 11.9).
+//   * A row-major W goes there unless
+//     - one row: 512-column blocks fill the CUs (3072 x 5632 11.9 / 13.7, 2048 x 5632
+//       11.7 / 10.1, 4096 x 4096 11.1 / 12.4, 11008 x 4096 18.2 / 22.3); two: from 2^25
+//       weights (4096 x 8192 17.6 / 19.2, 7168 x 4096 17.3 / 17.3, 6144 x 2048 11.0 / 12.2);
+//     - up to 16 rows, 128 and more 64-column strips: M = 4 / 16, 8192 x 2048 12.2 / 13.2
+//       against 13.0 / 13.5, 11008 x 4096 20.2 / 22.8 against 22.4 / 22.9, 14336 x 4096 26.7 /
+//       27.7 against 25.2 / 26.5.  (Not everywhere the faster one: 8192 x 4096 21.2 / 23.9
+//       against 18.6 / 19.3; 16384 x 8192 56 / 56 against 49 / 51.)
+//     - fewer strips whose K splits are one round of loads for the 8 waves (1024
+//       rows) and one work-group per CU: 6144 x 2048 9.8 / 11.2 against 12.2 / 12.6, 2048
+//       x 4096 7.7 / 9.2 against 8.7 / 8.9; not 6144 x 3072 (a second round, half empty)
+//       14.5 / 16.4 against 13.9 / 14.5, 5120 x 4096 (320 work-groups) 17.5 / 19.9
+//       against 14.8 / 15.2.
+static bool tiles_faster(const GemvArgs &a, bool wcol, bool rows, bool strip) {
+    const int64_t M = a.M, N = a.N, K = a.K;
+    if (M <= 16 && K <= 128 && (wcol ? K < 128 || N > 16384 : !rows || M * K <= 64)) return false;
     if (wcol) return true;
-    return !((N >= 8192 && M <= 16) || (M == 1 && N >= 2048 && (N >= 4096 || K <= 4096)));
+    if (N >= 8192) return M > 16;
+    if (M == 1) return !(N >= 2048 && (N >= 3072 || K <= 4096));
+    if (M == 2) return !(rows && N >= 4096 && N * K >= (1 << 25));
+    const int s = strip_splits(N, K);
+    return !(strip && K <= 1024 * s && cdiv(N, kStripW) * s <= num_cus() && (M <= 8 || (M <= 16 && K <= 2048)));
 }
 
 template <typename T, typename Tout>
@@ -841,7 +862,7 @@ static int gemv_run(int64_t M, int64_t N, int64_t K, int in_dtype, const void *x
         a.counters = reinterpret_cast<unsigned *>(workspace);
         a.partial = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + kGemvCounterBytes);
     }
-    if (splits <= 0 && tiles_faster(M, N, K, wcol) && (!bias || out_dtype == in_dtype)) {
+    if (splits <= 0 && tiles_faster(a, wcol, rows, strip) && (!bias || out_dtype == in_dtype)) {
         // (the partials behind the counters, within the size the query gives)
         const size_t most = gemv_workspace_bytes(M, N, K);
         const size_t have = workspace && aligned16(workspace) ? (workspace_bytes < most ? workspace_bytes : most) : 0;

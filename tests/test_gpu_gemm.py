@@ -420,6 +420,25 @@ def test_decode_gemm_ragged_k_and_splits(cuda, M, N, K):
         np.testing.assert_allclose(npy(o32), O.mm(npy(x), npy(W)), rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("layout", ["row", "col"])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 72, 8), (1, 512, 64), (1, 520, 72), (2, 520, 32), (2, 1000, 40), (3, 200, 128), (16, 136, 120), (16, 16392, 128),
+    (16, 136, 136), (17, 136, 64),                                                  # K up to 128, and one past
+    (1, 3072, 4616), (1, 3064, 4616), (2, 4096, 8192), (2, 4096, 8184),             # rows of 512 columns
+    (3, 2048, 4096), (8, 3072, 4096), (9, 3072, 4096), (16, 4160, 2048), (17, 4160, 2048), (8, 4096, 2056), (4, 4104, 4096)])  # strips
+def test_decode_gemm_route_lines(cuda, layout, M, N, K):
+    """Both sides of the lines between the decode GEMM's kernels; bias and fp32
+    output.  Whole numbers with sums below 2^24: fp32 results are exact, bf16
+    ones their rounding."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x, W, b = (torch.randint(-4, 5, s, generator=g).to(torch.bfloat16) for s in ((M, K), (K, N), (N,)))
+    Wd = W.to(cuda) if layout == "row" else W.t().contiguous().to(cuda).t()
+    want = (x.double() @ W.double()).float()
+    assert torch.equal(ops.mm(x.to(cuda), Wd, out_dtype=torch.float32).cpu(), want)
+    assert torch.equal(ops.mm(x.to(cuda), Wd).cpu(), want.to(torch.bfloat16))
+    assert torch.equal(ops.addmm(b.to(cuda), x.to(cuda), Wd).cpu(), (want + b.float()).to(torch.bfloat16))
+
+
 def test_decode_gemm_split_sequence_keeps_counters_zero(cuda):
     """Row-major decode GEMMs whose K split is summed by the last-arriving
     work-group of each strip: alternating shapes (different split counts and
