@@ -31,6 +31,7 @@
 // Semantics: aten scaled_dot_product_attention (the reference's fallthrough,
 // kuipy/kuiops.py:627-681 rejects is_causal; tests/test_jit_ops.py:173-193).
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_decode.hpp"
 
@@ -488,9 +489,9 @@ __global__ __launch_bounds__(128) void fa_decode_combine_kernel(AttnArgs a) {
 //     count (16384 unlikely keys: 2^-16), so that is done only in a second
 //     pass over the wave's keys, made when the first one's sums are not finite.
 // Against two rounded halves (2^-17 for bf16, and for f16 2^-25 of the largest)
-// it takes 0-4% longer in bf16, up to 7% in f16 (us: 16 sequences of 4000 keys
-// 43.5 / 43.7 / 44.2, 8 of 1024 11.5 / 11.8 / 12.3, head dim 64, 64 of 640 15.5 /
-// 16.0 / 16.2).
+// it takes 0-4% longer in bf16, up to 7% in f16 and there 13% for caches of a step
+// or two (us: 16 sequences of 4000 keys 43.5 / 43.7 / 44.2, 8 of 1024 11.5 / 11.8 /
+// 12.3, head dim 64, 64 of 640 15.5 / 16.0 / 16.2, 64 of 64 5.9 / 6.0 / 6.6).
 template <typename T> struct ProbSplit;
 template <> struct ProbSplit<bf16_t> {
     typedef bf16_t t2 __attribute__((ext_vector_type(2)));
@@ -897,9 +898,16 @@ static int64_t decode_chunk(int64_t s) {
 // empty and the VALU form has little to do), key rows whose byte offsets fit 31
 // bits and V rows that do not overlap (its V descriptor ends at the last key, so
 // past it a row that begins earlier, as in an expanded V, would still be read);
-// else up to 8.
+// else up to 8.  Caches of one step (64 keys of 128) for 3 or 4 rows in more
+// groups than fit the CUs at once are left to the VALU form too: the MFMA form's
+// 3 steps in flight are then mostly empty, and its 64 KB of tiles a work-group
+// cost a round (us, VALU against MFMA, capacities of 16 / 64 / 128 keys, bf16: 2048
+// groups 18.2 / 23.6 / 32.8 against 23.3 / 27.3 / 33.5, f16 18.0 / 23.3 / 32.9 against
+// 25.4 / 29.2 / 36.0; 400 groups within 6%).
 constexpr int kMfmaRows = 16;
-static int decode_rows_per_group(int64_t s, int64_t hd, int rows_kv, int64_t sk2, int64_t sv2) {
+static int decode_rows_per_group(int64_t s, int64_t hd, int rows_kv, int64_t sk2, int64_t sv2, int64_t kv_heads, bool f16) {
+    if (rows_kv == 3 || rows_kv == 4)
+        if (hd == 128 && kv_heads > 2 * (int64_t)num_cus() && s <= (f16 ? 128 : 64)) return 4;
     const int64_t st = sk2 > sv2 ? sk2 : sv2;
     if (rows_kv >= 3 && s < (1 << 30) && sk2 >= 0 && sv2 >= hd && (s + 64) * st * 2 < ((int64_t)1 << 31)) return kMfmaRows;
     return rows_kv <= 1 ? 1 : rows_kv <= 2 ? 2 : rows_kv <= 4 ? 4 : 8;
@@ -1011,7 +1019,7 @@ static int launch_decode(AttnArgs a, hipStream_t st) {
                            dim3(kDecodeWideWaves * 64), 0, st, a);
         return launch_status();
     }
-    const int R = decode_rows_per_group(a.s, HD, rows_kv, a.sk2, a.sv2);
+    const int R = decode_rows_per_group(a.s, HD, rows_kv, a.sk2, a.sv2, a.n * a.hkv, std::is_same<T, f16_t>::value);
     a.rows_per_group = R;
     a.row_groups = (int)cdiv(rows_kv, R);
     dim3 grid((unsigned)a.splits, (unsigned)(a.hkv * a.row_groups), (unsigned)a.n);
@@ -1125,7 +1133,7 @@ extern "C" int kuiops_sdpa_decode(int64_t n, int64_t hq, int64_t hkv, int64_t l,
     fill_args(a, n, hq, hkv, l, s, Q, sq, K, sk, V, sv, O, so, lse, scale, causal);
     a.kv_len = kv_len;
     const int64_t ss = s > 0 ? s : 1;
-    const int R = decode_rows_per_group(s, ev, (int)((hq / hkv) * l), a.sk2, a.sv2);
+    const int R = decode_rows_per_group(s, ev, (int)((hq / hkv) * l), a.sk2, a.sv2, n * hkv, dtype == KUIOPS_F16);
     a.chunk = decode_chunk_for(ss, n * hkv * cdiv((hq / hkv) * l, R), R == kMfmaRows ? 1 : 2);
     if (decode_row_wide(ss, ev, n * hq * l) || decode_single_split(ss, ev, R)) a.chunk = ss;
     a.splits = (int)cdiv(ss, a.chunk);

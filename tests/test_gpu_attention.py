@@ -208,7 +208,8 @@ def test_sdpa_decode_vs_oracle(cuda, n, hq, hkv, l, s, d):
 @pytest.mark.parametrize("n,hq,hkv,l,s,d", [
     (2, 6, 2, 1, 1300, 64), (1, 40, 2, 1, 1025, 128),      # 3 rows; 20 rows: two row groups
     (3, 8, 2, 4, 800, 128), (9, 32, 8, 1, 900, 128),       # 16 rows of 4 queries; 32 keys and one more per wave
-    (130, 16, 4, 1, 161, 64), (16, 8, 2, 1, 5000, 128)])   # one split; sixteen
+    (130, 16, 4, 1, 161, 64), (16, 8, 2, 1, 5000, 128),    # one split; sixteen
+    (257, 6, 2, 1, 64, 128), (257, 8, 2, 1, 65, 128), (130, 12, 4, 1, 128, 128), (260, 4, 2, 2, 129, 128)])   # short caches: the lines to the vector kernel
 def test_sdpa_decode_mfma_rows(cuda, dtype, n, hq, hkv, l, s, d):
     """Grouped-query decode on the MFMA kernel: device key counts from 0 to
     the capacity with NaN in the cache past them, query rows that do not fill
