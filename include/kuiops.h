@@ -104,6 +104,13 @@ KUIOPS_API const char *kuiops_status_string(int status);
  * stream.                                                                  */
 KUIOPS_API size_t kuiops_query_workspace(int op, int64_t a, int64_t b, int64_t c);
 
+/* The output tile (bm x bn) and the number of K splits that a bf16 / f16
+ * mm / addmm (batch = 1) or bmm of contiguous, 16-byte aligned operands runs
+ * with, given the workspace it asks for and no addend; 256 x 256 stands for
+ * the large-tile kernels.  Launches nothing and needs no GPU.              */
+KUIOPS_API int kuiops_query_gemm_tile(int64_t batch, int64_t M, int64_t K, int64_t N, int b_layout, int *bm,
+                                      int *bn, int *splits);
+
 /* ---------------------------------------------------------------- GEMM --
  * C[M, N] = A[M, K] @ B[K, N]
  * Replaces the mm launcher `(M, N, K, A, B, C)` of

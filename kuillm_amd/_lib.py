@@ -48,6 +48,8 @@ SIGNATURES = {
     "kuiops_abi_version": (_int, []),
     "kuiops_status_string": (ctypes.c_char_p, [_int]),
     "kuiops_query_workspace": (_sz, [_int, _i64, _i64, _i64]),
+    "kuiops_query_gemm_tile": (_int, [_i64, _i64, _i64, _i64, _int, ctypes.POINTER(_int), ctypes.POINTER(_int),
+                                      ctypes.POINTER(_int)]),
     "kuiops_mm": (_int, [_i64, _i64, _i64, _int, _vp, _i64, _vp, _i64, _int, _int, _vp, _i64, _vp]),
     "kuiops_addmm": (_int, [_i64, _i64, _i64, _dbl, _dbl, _int, _vp, _i64, _vp, _i64, _int,
                             _vp, _int, _i64, _int, _vp, _i64, _int, _vp, _sz, _vp]),

@@ -1293,9 +1293,9 @@ static int max_splits(int64_t M, int64_t N, int64_t K) {
 // weights streaming from HBM (us): 64 x 64 0.29 (one work-group per CU) and
 // 0.23 (several), 128 x 64 0.79 for 128 k, 128 x 128 0.59, 128 x 192 0.80,
 // 128 x 256 0.93.  Measured at 512 x N x K (bf16, nn.Linear weights cold in
-// HBM; the register-staged 128 x 128 tiles that ran here before, and this
-// choice): 11264 x 2048 47 -> 31.5 us, 2048 x 2048 30 -> 11.9, 2048 x 5632
-// 33 -> 27; 203 x 4864 x 896 24.9 -> 9.7.
+// HBM, in a replayed graph; the register-staged 128 x 128 tiles that ran here
+// before, and this choice): 11264 x 2048 49 -> 32 us, 2048 x 2048 20.8 -> 9.9, 2048 x
+// 5632 38 -> 27; 203 x 4864 x 896 19.9 -> 8.6 (a call with its bias 24.8 -> 10.9).
 struct TileCfg { int bm, bn, bk; float stage, stage_many; };
 static const TileCfg kTiles[] = {
     {64, 64, 64, 0.285f, 0.23f}, {128, 64, 128, 0.79f, 0.86f}, {128, 128, 64, 0.59f, 0.59f},
@@ -1401,19 +1401,34 @@ static bool dma_eligible(const GemmArgs &a, int64_t batch, bool bcol) {
            cdiv(a.M, 256) * cdiv(a.N, 256) * batch >= 128 && cdiv(a.M, 256) * cdiv(a.N, 256) * batch < INT32_MAX;
 }
 
+// The 256x256 tiles run 1.45 us per 64 k and about 5 us around them, one per CU:
+// with 128 of them (2048 x 4096 outputs) half the CUs idle and 128 x 256 tiles
+// finish first (K = 4096: 68-72 against 97-100 us, operands cold in HBM), with 256
+// or more they win (4096^3: 110-112 against 126-131 us).
+static bool large_tiles(const GemmArgs &a, int64_t batch, bool bcol, const TileChoice &tc) {
+    if (!dma_eligible(a, batch, bcol)) return false;
+    const int64_t tiles256 = cdiv(a.M, 256) * cdiv(a.N, 256) * batch;
+    const float us256 = 2.2f + (float)cdiv(tiles256, num_cus()) * ((float)(a.K / 64) * 1.45f + 3.f);
+    return gemm_kernel_choice() == 1 || a.K < 512 || us256 <= tc.us;
+}
+
+// Short K (64 or 128), full 256x256 tiles, several tiles per CU: the persistent
+// kernel overlaps each tile's output stores with the next tile's loads.
+static bool stream_tiles(const GemmArgs &a, int64_t batch, bool bcol) {
+    const int64_t lim = (int64_t)1 << 30;
+    const int64_t total = (a.M / 256) * (a.N / 256) * batch;
+    return gemm_kernel_choice() != 1 && (a.K == 64 || a.K == 128) && a.c_kind == KUIOPS_C_NONE && a.M % 256 == 0 &&
+           a.N % 256 == 0 && 256 * a.lda + a.K < lim && (bcol ? 256 * a.ldb + a.K : a.K * a.ldb + 256) < lim &&
+           a.lda % 8 == 0 && a.ldb % 8 == 0 && a.stride_a % 8 == 0 && a.stride_b % 8 == 0 && a.ldo % 8 == 0 &&
+           a.stride_o % 8 == 0 && aligned16(a.out) && total >= 2 * (int64_t)num_cus() && total < INT32_MAX;
+}
+
 template <typename T, typename Tout>
 static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int splits_req, void *ws, size_t ws_bytes,
                     hipStream_t st, bool any_ws = false) {
     if constexpr (sizeof(Tout) == 2) {
-        // short K (64 or 128), full 256x256 tiles, several tiles per CU: the
-        // persistent kernel overlaps each tile's output stores with the next
-        // tile's loads
-        const int64_t lim = (int64_t)1 << 30;
         const int64_t total = (a.M / 256) * (a.N / 256) * batch;
-        if (aligned && splits_req <= 1 && gemm_kernel_choice() != 1 && (a.K == 64 || a.K == 128) &&
-            a.c_kind == KUIOPS_C_NONE && a.M % 256 == 0 && a.N % 256 == 0 && 256 * a.lda + a.K < lim &&
-            (bcol ? 256 * a.ldb + a.K : a.K * a.ldb + 256) < lim && a.lda % 8 == 0 && a.ldb % 8 == 0 && a.stride_a % 8 == 0 && a.stride_b % 8 == 0 && a.ldo % 8 == 0 &&
-            a.stride_o % 8 == 0 && aligned16(a.out) && total >= 2 * (int64_t)num_cus() && total < INT32_MAX) {
+        if (aligned && splits_req <= 1 && stream_tiles(a, batch, bcol)) {
             a.tiles_m = (int)(a.M / 256);
             a.tiles_n = (int)(a.N / 256);
             a.vec_store = true;
@@ -1440,13 +1455,7 @@ static int run_mfma(GemmArgs a, int64_t batch, bool bcol, bool aligned, int spli
     }
     const TileChoice tc = choose_tile(a.M, a.N, a.K, batch, ws_ok ? max_s : 1,
                                       batch == 1 ? splits_req : 1);
-    // The 256x256 tiles run 1.45 us per 64 k and about 5 us around them, one
-    // per CU: with 128 of them (2048 x 4096 outputs) half the CUs idle and
-    // 128 x 256 tiles finish first (K = 4096: 60 against 98 us), with 256 or
-    // more they win (4096^3: 98 against 122 us).
-    const int64_t tiles256 = cdiv(a.M, 256) * cdiv(a.N, 256) * batch;
-    const float us256 = 2.2f + (float)cdiv(tiles256, num_cus()) * ((float)(a.K / 64) * 1.45f + 3.f);
-    if (aligned && splits_req <= 1 && dma_eligible(a, batch, bcol) && (gemm_kernel_choice() == 1 || a.K < 512 || us256 <= tc.us)) {
+    if (aligned && splits_req <= 1 && large_tiles(a, batch, bcol, tc)) {
         a.tiles_m = (int)cdiv(a.M, 256);
         a.tiles_n = (int)cdiv(a.N, 256);
         const int vec = sizeof(Tout) == 2 ? 8 : 4;    // elements per vector store
@@ -1655,6 +1664,30 @@ size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 }  // namespace kuiops
 
 using namespace kuiops;
+
+extern "C" int kuiops_query_gemm_tile(int64_t batch, int64_t M, int64_t K, int64_t N, int b_layout, int *bm, int *bn,
+                                      int *splits) {
+    if (batch < 1 || M < 1 || K < 1 || N < 1 || (b_layout != KUIOPS_B_ROW && b_layout != KUIOPS_B_COL) || !bm || !bn || !splits)
+        return KUIOPS_E_INVALID;
+    if (batch > 65535 || M > INT32_MAX / 2 || N > INT32_MAX / 2) return KUIOPS_E_UNSUPPORTED;
+    const bool bcol = b_layout == KUIOPS_B_COL;
+    GemmArgs a{};
+    a.M = M; a.N = N; a.K = K;
+    a.lda = K; a.ldb = bcol ? K : N; a.ldo = N;
+    a.stride_a = M * K; a.stride_b = K * N; a.stride_o = M * N;
+    if (!rows_aligned(a, bcol, batch) || !offsets_fit(a, bcol)) return KUIOPS_E_UNSUPPORTED;
+    const TileChoice tc = choose_tile(M, N, K, batch, batch == 1 ? max_splits(M, N, K) : 1, batch == 1 ? 0 : 1);
+    if (stream_tiles(a, batch, bcol) || large_tiles(a, batch, bcol, tc)) {
+        *bm = *bn = 256;
+        *splits = 1;
+        return KUIOPS_OK;
+    }
+    const TileCfg &t = kTiles[tc.tile];
+    *bm = t.bm;
+    *bn = t.bn;
+    *splits = (int)cdiv(K, cdiv(cdiv(K, tc.splits), t.bk) * t.bk);
+    return KUIOPS_OK;
+}
 
 extern "C" int kuiops_mm(int64_t M, int64_t N, int64_t K, int in_dtype, const void *A, int64_t lda,
                          const void *B, int64_t ldb, int b_layout, int out_dtype, void *C, int64_t ldc,

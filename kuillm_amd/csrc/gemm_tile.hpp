@@ -117,7 +117,7 @@ __device__ __forceinline__ int swz_brow(int k) {
 // were within 5% of this form; larger tiles are what helps, and K splits where
 // they leave CUs idle.  Register-staged tiles of the same size
 // (gemm_mfma_kernel) wait for a whole load latency per stage: 512 x 11264 x
-// 2048 47 -> 31.5 us.
+// 2048 49 -> 32 us.
 template <typename T, bool BCOL, typename Tout, int WM, int WN, int WK, int TM, int TN, int NS, bool SPLIT>
 __global__ __launch_bounds__(WM * WN * WK * 64) void gemm_tile_kernel(GemmArgs a) {
     constexpr int NW = WM * WN * WK;                 // waves

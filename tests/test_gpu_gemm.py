@@ -6,6 +6,8 @@ Tolerance (north star): bf16 / f16 results within rel 1e-2 / abs 1e-2 of the
 fp32-accumulate oracle, elementwise: |out - ref| <= 1e-2 + 1e-2 * |ref|.
 fp32 results: allclose(rtol=1e-3, atol=1e-3) as the reference's tests
 (tests/test_jit_ops.py:34-43)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -116,7 +118,8 @@ def test_mm_closed_forms(cuda):
 
 
 # Shapes that take the 4-wave 256x256 kernel (K % 128 == 0, K >= 512, at
-# least 128 tiles) with partial edge tiles in M and N.
+# least 128 tiles) with partial edge tiles in M and N (row-major, the first one's
+# 4100 columns are odd strides: 128x128 tiles of gemm_mfma_kernel).
 WAVE_SHAPES = [(2000, 4100, 640), (4096, 2056, 512), (1288, 6400, 1024)]
 
 
@@ -137,22 +140,34 @@ def test_addmm_wave_kernel_edges(cuda, layout, M, N, K, kind):
     assert_tol(out, O.addmm(npy(C), npy(A), npy(B), alpha, beta), torch.bfloat16)
 
 
-# One shape per output tile of the tile kernel (64x64, 128x64, 128x128,
-# 128x192, 128x256), each with ragged last tiles, K remainders of 8 .. 56 and
-# fewer, as many or more K steps than LDS stages; split K (130 x 384, 5 K
-# ranges); an output whose rows are not 16-byte aligned (N = 1003).
-TILE_SHAPES = [(65, 136, 8), (200, 520, 264), (300, 5000, 1032), (1000, 4000, 200), (500, 11264, 136),
-               (2100, 4104, 216), (130, 384, 2568), (257, 1003, 1160)]
+def gemm_tile(batch, M, K, N, layout="row"):
+    """(bm, bn, K splits) that the library runs such a product with."""
+    got = [ctypes.c_int() for _ in range(3)]
+    b = _lib.B_ROW if layout == "row" else _lib.B_COL
+    _lib.check("kuiops_query_gemm_tile", _lib.load().kuiops_query_gemm_tile(batch, M, K, N, b, *map(ctypes.byref, got)))
+    return tuple(v.value for v in got)
+
+
+# Every output tile of the tile kernel, with ragged last tiles, K remainders of
+# 8 .. 56 and fewer, as many or more K steps than LDS stages; split K of each
+# tile that splits; an output whose rows are not 16-byte aligned (N = 1003).
+TILE_SHAPES = [((65, 136, 8), (64, 64, 1)), ((200, 520, 264), (64, 64, 1)), ((300, 5000, 1032), (128, 64, 1)),
+               ((1000, 4000, 200), (128, 128, 1)), ((500, 11264, 136), (128, 192, 1)), ((2100, 4104, 216), (128, 192, 1)),
+               ((130, 384, 2568), (64, 64, 5)), ((257, 1003, 1160), (64, 64, 1)),
+               ((519, 9936, 200), (128, 256, 1)), ((519, 9936, 456), (128, 256, 1)),
+               ((66, 2712, 2272), (128, 64, 4)), ((68, 4168, 2696), (128, 128, 5)), ((132, 5600, 3768), (128, 192, 3))]
 
 
 @pytest.mark.parametrize("layout", ["row", "col"])
-@pytest.mark.parametrize("M,N,K", TILE_SHAPES)
-def test_addmm_tile_kernel_edges(cuda, layout, M, N, K):
+@pytest.mark.parametrize("shape,tile", TILE_SHAPES)
+def test_addmm_tile_kernel_edges(cuda, layout, shape, tile):
     """Bias and full addends, fp32 output, both B layouts.  |error| <= half a
     bf16 ulp (2^-9 |ref|) plus fp32 sums of K products of size ~0.05
     (K * 2^-24 * 0.2 < 1e-4), inside the file's 1e-2."""
+    M, N, K = shape
     if layout == "row" and N % 8:
         pytest.skip("row-major B of odd width is another kernel")
+    assert gemm_tile(1, M, K, N, layout) == tile
     A, B = gen((M, K), torch.bfloat16, seed=51), gen((K, N), torch.bfloat16, 0.05, seed=52)
     bias, C = gen((N,), torch.bfloat16, seed=53), gen((M, N), torch.bfloat16, seed=54)
     Bd = B.to(cuda) if layout == "row" else B.t().contiguous().to(cuda).t()
@@ -355,9 +370,13 @@ def test_bmm_golden(cuda, golden, dtype):
 
 
 @pytest.mark.parametrize("b,M,K,N", [(4, 64, 64, 64), (3, 130, 72, 200), (2, 256, 128, 512),
-                                     (8, 1024, 640, 1024),     # batched 4-wave kernel (K >= 512)
+                                     (8, 1024, 640, 1024),     # 128x256 tiles
+                                     (10, 1020, 640, 1016),    # batched 4-wave kernel (K >= 512), ragged tiles
+                                     (300, 130, 72, 56),       # more 64x64 tiles than CUs, few columns
                                      (6, 600, 128, 1800)])     # short-K 8-wave kernel, ragged tiles
 def test_bmm_vs_oracle(cuda, b, M, K, N):
+    if M > 1000:
+        assert gemm_tile(b, M, K, N) == ((128, 256, 1) if M == 1024 else (256, 256, 1))
     A, B = gen((b, M, K), torch.bfloat16, seed=9), gen((b, K, N), torch.bfloat16, seed=10)
     assert_tol(ops.bmm(A.to(cuda), B.to(cuda)), O.bmm(npy(A), npy(B)), torch.bfloat16)
     # a K-contiguous B (transposed view) gives the same result
