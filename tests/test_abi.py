@@ -250,3 +250,19 @@ def test_decode_rows_workspace_follows_the_device(monkeypatch):
     for _ in lib.sizes:
         ops.decode_rows_batched(x, W)
     assert lib.given == lib.sizes
+
+
+def test_query_gemm_tile(lib):
+    bm, bn, splits = (ctypes.c_int() for _ in range(3))
+
+    def tile(batch, M, K, N, layout=_lib.B_ROW):
+        status = lib.kuiops_query_gemm_tile(batch, M, K, N, layout, bm, bn, splits)
+        return (bm.value, bn.value, splits.value) if status == _lib.OK else status
+
+    assert tile(1, 4096, 4096, 4096) == (256, 256, 1)
+    assert tile(32, 2048, 128, 2048) == (256, 256, 1)
+    assert tile(1, 65, 8, 136) == (64, 64, 1)
+    assert tile(1, 128, 8192, 128)[2] > 1 and tile(2, 128, 8192, 128)[2] == 1
+    assert tile(1, 100, 8, 101) == _lib.E_UNSUPPORTED and tile(1, 100, 8, 101, _lib.B_COL) == (64, 64, 1)
+    assert tile(1, 100, 12, 104) == _lib.E_UNSUPPORTED
+    assert tile(0, 1, 8, 8) == tile(1, 8, 8, 0) == tile(1, 8, 8, 8, 7) == _lib.E_INVALID
