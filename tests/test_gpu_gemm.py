@@ -458,6 +458,28 @@ def test_decode_gemm_route_lines(cuda, layout, M, N, K):
     assert torch.equal(ops.addmm(b.to(cuda), x.to(cuda), Wd).cpu(), (want + b.float()).to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("layout", ["row", "col"])
+@pytest.mark.parametrize("splits", [0, 3])
+@pytest.mark.parametrize("M,N,K", [(2, 1000, 1032), (17, 8200, 264), (33, 4160, 2048), (50, 8200, 1096), (64, 200, 520)])
+def test_decode_gemm_f32_out_with_bias(cuda, layout, splits, M, N, K):
+    """fp32 output with a bias, and a caller's split count, which the tile kernel
+    does not take: rows, strips of 17 to 64 rows (two to four MFMA blocks), and
+    the split-K kernel in both layouts.  Whole numbers: exact."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x, W, b = (torch.randint(-4, 5, s, generator=g).to(torch.bfloat16).to(cuda) for s in ((M, K), (K, N), (N,)))
+    Wd = W if layout == "row" else W.t().contiguous()
+    lib = _lib.load()
+    # (three splits' partials: more than the size for a split count of the library's)
+    nbytes = max(lib.kuiops_query_workspace(_lib.OP_GEMV_SPLITK, M, N, K), 16384 + 3 * M * N * 4)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=cuda)
+    out = torch.full((M, N), float("nan"), device=cuda)
+    _lib.check("kuiops_gemv_splitk", lib.kuiops_gemv_splitk(
+        M, N, K, _lib.BF16, x.data_ptr(), K, Wd.data_ptr(), Wd.stride(0), _lib.B_ROW if layout == "row" else _lib.B_COL,
+        b.data_ptr(), _lib.F32, out.data_ptr(), N, splits, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out.cpu().double(), x.cpu().double() @ W.cpu().double() + b.cpu().double())
+    assert not ws[:16384].any()
+
+
 def test_decode_gemm_split_sequence_keeps_counters_zero(cuda):
     """Row-major decode GEMMs whose K split is summed by the last-arriving
     work-group of each strip: alternating shapes (different split counts and
