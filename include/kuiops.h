@@ -405,7 +405,8 @@ KUIOPS_API int kuiops_index_multi(int64_t outer, int k, const int64_t *sizes, in
 /* RMSNorm with an optional fused residual add, per row of [m, n]:
  *   h = x (+ residual)      res_out = h (if non-null; may equal residual)
  *   y = weight * round(h * rsqrt(mean(h^2) + eps)),  n <= 8192.
- * Rows of residual and res_out must not overlap (ldr = 0: one row for all).
+ * Rows of res_out must not overlap; those of residual may (ldr = 0: one row
+ * for all).
  * Replaces the reference's elementwise chain pow / mean.dim / add / rsqrt /
  * mul (ElementwiseImpl kuipy/kuiops.py:150-320, MeanImpl :860-921), one
  * launch per aten op there.                                                */

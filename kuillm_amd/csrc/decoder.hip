@@ -991,8 +991,8 @@ extern "C" int kuiops_rmsnorm(int64_t m, int64_t n, int dtype, const void *x, in
     if (m == 0 || n == 0) return KUIOPS_OK;
     if (!x || !weight || !y) return KUIOPS_E_INVALID;
     if (dtype != KUIOPS_BF16 && dtype != KUIOPS_F16) return KUIOPS_E_UNSUPPORTED;
-    // rows that overlap (a residual of row stride 0 is one row for all)
-    if (m > 1 && ((residual && ldr != 0 && ldr < n) || (res_out && ldro < n))) return KUIOPS_E_INVALID;
+    // written rows that overlap (a residual is only read: its rows may)
+    if (m > 1 && res_out && ldro < n && ldro > -n) return KUIOPS_E_INVALID;
     if (n % 8 || ldx % 8 || ldy % 8 || (residual && ldr % 8) || (res_out && ldro % 8)) return KUIOPS_E_UNSUPPORTED;
     if (!aligned16(x) || !aligned16(weight) || !aligned16(y) || (residual && !aligned16(residual)) ||
         (res_out && !aligned16(res_out)))

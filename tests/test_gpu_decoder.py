@@ -50,6 +50,18 @@ def test_rmsnorm_vs_oracle(cuda, m, n):
     close(f(y2), ry2)
 
 
+@pytest.mark.parametrize("ldr", [0, 8, 248])
+def test_rmsnorm_overlapping_residual_rows(cuda, ldr):
+    """A residual's rows may overlap, or be one row for all: they are only read."""
+    m, n = 9, 256
+    x, w, store = bf((m, n), 4), bf((n,), 5), bf((ldr * (m - 1) + n,), 6)
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=cuda)
+    y = ops.rmsnorm(x.to(cuda), w.to(cuda), 1e-5, residual=store.to(cuda).as_strided((m, n), (ldr, 1)), res_out=out)
+    ry, rh = O.rmsnorm(f(x), f(w), 1e-5, residual=f(store.as_strided((m, n), (ldr, 1))))
+    np.testing.assert_array_equal(f(out), rh)
+    close(f(y), ry)
+
+
 @pytest.mark.parametrize("m,n", [(1, 5632), (64, 512), (3, 8)])
 def test_silu_mul_vs_oracle(cuda, m, n):
     gu = bf((m, 2 * n), 4, 2.0)
