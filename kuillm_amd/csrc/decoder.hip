@@ -1052,7 +1052,8 @@ extern "C" int kuiops_rope_kv_append(int64_t n, int64_t t, int64_t hq, int64_t h
     // 400 2.4 / 3.0, 4000 4.6 / 5.1), and tokens enough for their rows (head dim 256,
     // 32 + 8 heads: 128 tokens 4.5 / 4.8, 200 5.8 / 5.4).
     const int64_t heads = hq + 2 * hkv;
-    const bool by_token = n * t >= (hd > 128 ? 192 : 128) && heads >= 4 && n * t * heads >= 3000;
+    // (a launch of 2^32 threads along x wraps around)
+    const bool by_token = n * t >= (hd > 128 ? 192 : 128) && heads >= 4 && n * t * heads >= 3000 && t < (1 << 24);
     const auto aligned8 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
     if (by_token && hd / 2 <= kRopeMaxHalf && !(sq[0] % 4 || sq[1] % 4 || sq[2] % 4 || sk[0] % 4 || sk[1] % 4 || sk[2] % 4) &&
         aligned8(q_out) && aligned8(k_cache)) {

@@ -312,6 +312,28 @@ def test_decode_gate_up_matches_unfused(cuda, ffn, K):
     close(f(out), O.silu_mul(np.concatenate([g, u], -1))[0])
 
 
+def test_rope_kv_append_more_tokens_than_a_launch(cuda):
+    """2^24 tokens and some: at 256 threads a token a launch along x would wrap
+    around.  The last tokens are what a call of their own gives."""
+    t, hq, hkv, hd, k = (1 << 24) + 3, 2, 1, 8, 5
+    qkv = torch.zeros(1, t, (hq + 2 * hkv) * hd, dtype=torch.bfloat16, device=cuda)
+    qkv[:, :k], qkv[:, -k:] = bf((1, k, qkv.shape[2]), 8).to(cuda), bf((1, k, qkv.shape[2]), 9).to(cuda)
+    inv = torch.tensor(O.rope_inv_freq(hd, 10000.0)).to(cuda)
+
+    def run(rows, cap, pos):
+        n = rows.shape[1]
+        q = torch.zeros(1, hq, n, hd, dtype=torch.bfloat16, device=cuda)
+        kc = torch.zeros(1, hkv, cap, hd, dtype=torch.bfloat16, device=cuda)
+        vc = torch.zeros_like(kc)
+        ops.rope_kv_append(rows, hq, hkv, hd, inv, torch.tensor([pos], dtype=torch.int32, device=cuda), q, kc, vc)
+        return q, kc, vc
+    q, kc, vc = run(qkv, t, 0)
+    for at in (0, t - k):
+        wq, wk, wv = run(qkv[:, at:at + k], t, at)
+        assert torch.equal(q[:, :, at:at + k], wq)
+        assert torch.equal(kc[:, :, at:at + k], wk[:, :, at:at + k]) and torch.equal(vc[:, :, at:at + k], wv[:, :, at:at + k])
+
+
 @pytest.mark.parametrize("hq,hkv,hd,K,pos", [(32, 8, 64, 2048, 517), (4, 2, 128, 256, 3), (8, 8, 64, 512, 0)])
 def test_decode_qkv_rope_matches_unfused(cuda, hq, hkv, hd, K, pos):
     """kuiops_decode_qkv_rope (rotary + cache-append epilogue, optional
