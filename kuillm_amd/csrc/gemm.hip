@@ -1303,20 +1303,44 @@ static const TileCfg kTiles[] = {
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 struct TileChoice { int tile, splits; float us; };
 
+// The same for the products of a batch, whose tiles are often mostly empty (their
+// rows and columns past the product cost no traffic) and many to a CU: a line
+// through the measured times of each tile, one for at most a tile per CU (us, and
+// us per stage) and one for more (us, then per tile and CU: us, us per stage, and us
+// per 1000 k of each row and column).  Over 1175 products (2-1500 of 1-4000 x
+// 8-3000 x 8-12000) it is 11% off a measured time (rms) and its choice 1.6% slower than the
+// best of the five; the sum of rounds above, which knows neither, 10%, and up to
+// twice as slow (us, that choice and this one: 800 x (8 x 304 x 72) 50.0 -> 28.5, 209 x (496
+// x 24 x 64) 16.6 -> 12.7, 60 x (8 x 1200 x 72) 15.9 -> 10.1).
+struct BatchCost { float one, one_stage, many, tile, stage, edge; };
+static const BatchCost kBatchCost[] = {{3.4f, 0.125f, 2.4f, 1.0f, 0.34f, 0.f}, {4.7f, 0.226f, 3.6f, 3.0f, 0.66f, 0.02f},
+                                       {4.5f, 0.203f, 3.8f, 2.6f, 0.58f, 0.017f}, {7.4f, 0.32f, 5.5f, 5.0f, 0.65f, 0.02f},
+                                       {5.6f, 0.42f, 4.7f, 3.4f, 0.76f, 0.026f}};
+
+static float batch_us(int t, int64_t M, int64_t N, int64_t K, int64_t batch) {
+    const TileCfg &c = kTiles[t];
+    const BatchCost &b = kBatchCost[t];
+    const int64_t tm = cdiv(M, c.bm), tn = cdiv(N, c.bn), tiles = tm * tn * batch, cus = num_cus();
+    const float stages = (float)cdiv(K, c.bk), m = (float)M / tm, n = (float)N / tn, k = (float)K * 1e-3f;
+    if (tiles <= cus) return b.one + stages * b.one_stage + k * (m + n) * 0.025f;
+    return b.many + (float)tiles / cus * (b.tile + stages * b.stage + k * (m + n) * b.edge + m * n * 5e-5f);
+}
+
 // The tile and split count of least estimated time: rounds of one tile per
 // CU, and for a split the partials' traffic plus the second launch.  max_s
-// bounds the splits; fixed_s > 0 asks for that many.  Up to 64 columns in more
-// 64x64 tiles than CUs, those are always fastest: two and more fit a CU, which the
-// model does not count, and larger ones share nothing (209 x (496 x 24), us for 64x64
-// / 128x64 / 128x128: K = 64 12.7 / 18.4 / 16.6, K = 512 30.4 / 35.7 / 35.6; 60000 x 64,
-// K = 128 9.3 / 11.0 / 10.9).
+// bounds the splits; fixed_s > 0 asks for that many.  A batch takes the tile
+// of batch_us where that is 10% ahead (the time stays the sum of rounds, which is
+// what the 256x256 tiles' is held against).  Up to 64 columns in more 64x64 tiles
+// than CUs always take those: two and more fit a CU, and larger ones share
+// nothing (us for 64x64 / 128x64 / 128x128: 60000 x 64, K = 128, 9.3 / 11.0 / 10.9, 209 x
+// (496 x 24), K = 512, 30.4 / 35.7 / 35.6).
 static TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int max_s, int fixed_s) {
     TileChoice best{0, 1, 1e30f};
     const int64_t cus = num_cus();
-    for (int t = 0; t < kNumTiles; ++t) {
+    const bool only64 = N <= 64 && cdiv(M, 64) * batch > cus;
+    for (int t = 0; t < (only64 ? 1 : kNumTiles); ++t) {
         const TileCfg &c = kTiles[t];
         const int64_t tiles = cdiv(M, c.bm) * cdiv(N, c.bn) * batch;
-        if (t > 0 && N <= 64 && cdiv(M, 64) * batch > cus) break;
         for (int s = fixed_s > 0 ? fixed_s : 1; s <= (fixed_s > 0 ? fixed_s : max_s); ++s) {
             const int64_t rounds = cdiv(tiles * s, cus);
             const int64_t stages = cdiv(cdiv(K, s), c.bk);
@@ -1324,6 +1348,12 @@ static TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, in
             if (s > 1) us += 4.f + (float)s * (float)(M * N) * 8.f / 6e6f;
             if (us < best.us) best = {t, s, us};
         }
+    }
+    if (batch > 1 && !only64) {
+        int b = 0;
+        for (int t = 1; t < kNumTiles; ++t)
+            if (batch_us(t, M, N, K, batch) < batch_us(b, M, N, K, batch)) b = t;
+        if (batch_us(best.tile, M, N, K, batch) > 1.1f * batch_us(b, M, N, K, batch)) best.tile = b;
     }
     return best;
 }

@@ -369,14 +369,16 @@ def test_bmm_golden(cuda, golden, dtype):
     assert_tol(out, O.bmm(npy(t("A")), npy(t("B"))), dtype)
 
 
-@pytest.mark.parametrize("b,M,K,N", [(4, 64, 64, 64), (3, 130, 72, 200), (2, 256, 128, 512),
-                                     (8, 1024, 640, 1024),     # 128x256 tiles
-                                     (10, 1020, 640, 1016),    # batched 4-wave kernel (K >= 512), ragged tiles
-                                     (300, 130, 72, 56),       # more 64x64 tiles than CUs, few columns
-                                     (6, 600, 128, 1800)])     # short-K 8-wave kernel, ragged tiles
-def test_bmm_vs_oracle(cuda, b, M, K, N):
-    if M > 1000:
-        assert gemm_tile(b, M, K, N) == ((128, 256, 1) if M == 1024 else (256, 256, 1))
+@pytest.mark.parametrize("b,M,K,N,tile", [
+    (4, 64, 64, 64, (64, 64)), (3, 130, 72, 200, (64, 64)), (2, 256, 128, 512, (64, 64)), (8, 1024, 640, 1024, (128, 256)),
+    (10, 1020, 640, 1016, (256, 256)),      # batched 4-wave kernel (K >= 512), ragged tiles
+    (6, 600, 128, 1800, (256, 256)),        # short-K 8-wave kernel, ragged tiles
+    # ragged tiles of a batch, up to one per CU
+    (42, 72, 72, 248, (128, 64)), (39, 11, 80, 712, (128, 128)), (55, 10, 336, 728, (128, 192)), (75, 10, 80, 672, (128, 256)),
+    # and more
+    (300, 130, 72, 56, (64, 64)), (90, 9, 200, 632, (64, 64)), (133, 197, 72, 72, (128, 128)), (119, 9, 72, 1016, (128, 256))])
+def test_bmm_vs_oracle(cuda, b, M, K, N, tile):
+    assert gemm_tile(b, M, K, N) == (*tile, 1)
     A, B = gen((b, M, K), torch.bfloat16, seed=9), gen((b, K, N), torch.bfloat16, seed=10)
     assert_tol(ops.bmm(A.to(cuda), B.to(cuda)), O.bmm(npy(A), npy(B)), torch.bfloat16)
     # a K-contiguous B (transposed view) gives the same result
