@@ -1622,18 +1622,19 @@ static bool rows_aligned(const GemmArgs &a, bool bcol, int64_t batch) {
 
 // 16-bit operands of odd strides whose K is so short that gemm_mfma_kernel's time
 // is its stage of 64 k, not its arithmetic: up to K = 16 always (its K tail is
-// loaded by elements), up to 32 for few tiles or ones that are mostly empty (and
-// the transposing of a row-major B is in vain), up to 48 for many of those (us,
-// SIMT against MFMA, row-major B: 9 x (5 x 59) K = 7 4.0 / 6.3, K = 21 5.8 / 6.2, K =
-// 41 7.6 / 6.1; 100 x (1 x 511) K = 25 9.3 / 11.4, K = 37 11.6 / 11.5; 209 x (496 x 23) K
-// = 7 10.1 / 22.3, K = 41 19.6 / 22.5, K = 64 24.5 / 20.0; 3000 x 5001 K = 8 21.5 /
-// 21.7, K = 31 34.2 / 29.4).
+// loaded by elements), up to 32 for few tiles, ones that are mostly empty (and
+// the transposing of a row-major B is in vain) or many that are not quite full, up
+// to 48 for many mostly empty ones (us, SIMT against MFMA, row-major B: 9 x (5 x 59) K =
+// 7 4.0 / 6.3, K = 21 5.8 / 6.2, K = 41 7.6 / 6.1; 100 x (1 x 511) K = 25 9.3 / 11.4, K = 37
+// 11.6 / 11.5; 233 x (55 x 321) K = 25 16.2 / 22.3; 209 x (496 x 23) K = 7 10.1 / 22.3, K = 41
+// 19.6 / 22.5, K = 64 24.5 / 20.0; 3000 x 5001 K = 8 21.5 / 21.7, K = 31 34.2 / 29.4;
+// K-contiguous: 802 x (6 x 1559) K = 19 89 / 169, 64 x (201 x 199) K = 21 13.3 / 12.5).
 static bool simt_faster(const GemmArgs &a, int64_t batch, bool bcol) {
     if (cdiv(a.M, 64) > 65535 * 32 || cdiv(a.N, 64) > 65535) return false;
     const int64_t tiles = cdiv(a.M, 64) * cdiv(a.N, 128) * batch;
-    const bool empty = a.N <= 32 && tiles > 2 * num_cus();
-    if (a.K > 32) return a.K <= 48 && empty && !bcol;
-    return a.K <= 16 || tiles <= 128 || empty || (!bcol && (a.N <= 64 || a.M <= 16));
+    const bool many = tiles > 2 * num_cus(), full = a.M * a.N * batch >= tiles * (64 * 128) / 10 * 9;
+    if (a.K > 32) return a.K <= 48 && a.N <= 32 && many && !bcol;
+    return a.K <= 16 || tiles <= 128 || (many && !full) || (!bcol && (a.N <= 64 || a.M <= 16));
 }
 
 // Shared entry for mm / addmm / bmm.

@@ -185,7 +185,7 @@ def test_addmm_tile_kernel_edges(cuda, layout, shape, tile):
                                      (3, 65, 16, 63), (2, 130, 15, 257), (32, 70, 32, 129), (300, 65, 48, 32), (260, 129, 47, 31),
                                      (200, 16, 31, 130), (160, 70, 29, 63),
                                      # one past each line
-                                     (260, 65, 17, 130), (2, 70, 33, 129), (300, 65, 49, 31), (300, 65, 47, 33), (33, 70, 31, 129)])
+                                     (260, 64, 17, 254), (100, 190, 31, 130), (2, 70, 33, 129), (300, 65, 49, 31), (300, 65, 47, 33), (33, 70, 31, 129)])
 @pytest.mark.parametrize("layout", ["row", "col"])
 def test_bmm_odd_strides(cuda, dtype, b, M, K, N, layout):
     """Rows of odd length at 2-byte alignment: slices of wider NaN-filled
