@@ -1309,7 +1309,7 @@ struct TileChoice { int tile, splits; float us; };
 // us per stage) and one for more (us, then per tile and CU: us, us per stage, and us
 // per 1000 k of each row and column).  Over 1175 products (2-1500 of 1-4000 x
 // 8-3000 x 8-12000) it is 11% off a measured time (rms) and its choice 1.6% slower than the
-// best of the five; the sum of rounds above, which knows neither, 10%, and up to
+// best of the five; the sum of rounds below, which knows neither, 10%, and up to
 // twice as slow (us, that choice and this one: 800 x (8 x 304 x 72) 50.0 -> 28.5, 209 x (496
 // x 24 x 64) 16.6 -> 12.7, 60 x (8 x 1200 x 72) 15.9 -> 10.1).
 struct BatchCost { float one, one_stage, many, tile, stage, edge; };
